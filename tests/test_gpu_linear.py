@@ -211,3 +211,53 @@ def test_weight_planes_layout():
     assert torch.equal(got, want)
     err = (x1.double() + x2.double() + x3.double() - w.double()).abs()
     assert bool((err <= 2.0 ** -24 * w.double().abs()).all())
+
+
+@pytest.mark.parametrize("form", ["f32", "planes", "bf16"])
+@pytest.mark.parametrize("m,n,k,extras", [
+    (65, 64, 32, "none"), (96, 640, 64, "bias"), (97, 384, 96, "residual"),     # fewer than 256 rows, 1-3 k tiles
+    (255, 128, 160, "bias_tanh"), (256, 64, 32, "none"), (257, 640, 64, "bias"),
+    (333, 640, 640, "residual"), (511, 5120, 128, "bias_sigmoid"), (1000, 128, 2560, "none"),
+    (130, 1091, 96, "bias"), (300, 1091, 640, "none"), (70, 36, 64, "residual"),  # columns no large tile fits
+])
+def test_small_tile_products(form, m, n, k, extras):
+    """gemm_ps_kernel at the edges of its tiles (32, 64 and 128 rows and columns),
+    of its load pipeline (fewer k tiles than buffers) and of its column range,
+    against float64.  The fp32 forms must stay within (K + 3) 2^-24 of sum |a||w|
+    (fp32 accumulation of K terms plus the three-part split's dropped terms),
+    the bf16 form within that plus its activation split's 2^-16; the epilogue
+    adds at most a few roundings of values of order 1."""
+    if form == "bf16" and n % 64 != 0 and n % 160 != 0:
+        pytest.skip("bf16 weights need N % 64 == 0 or N % 160 == 0 above 64 rows")
+    if form == "planes" and n % 16 != 0:
+        pytest.skip("planes need N % 16 == 0")
+    print(f"small tiles {form} {m}x{n}x{k} {extras}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(m * 11 + n + k)
+    a = torch.randn(m, k, generator=g).cuda()
+    w = (torch.randn(n, k, generator=g) * 0.05).cuda()
+    w = w.bfloat16() if form == "bf16" else w
+    bias = (torch.randn(n, generator=g) * 0.1).cuda() if "bias" in extras else None
+    act = 1 if "tanh" in extras else 2 if "sigmoid" in extras else 0
+    res = torch.randn(m, n, generator=g).cuda() if extras == "residual" else None
+    c = torch.full((m + 1, n), float("nan"), device="cuda")  # the row past the product must stay untouched
+    st = torch.cuda.current_stream().cuda_stream
+    tail = (None if bias is None else bias.data_ptr(), act, None if res is None else res.data_ptr(), c.data_ptr(), st)
+    if form == "planes":
+        planes = torch.empty(lib().yuf_x3_planes_elems(n, k), dtype=torch.int16, device="cuda")
+        check(lib().yuf_x3_split_planes(n, k, w.data_ptr(), planes.data_ptr(), st))
+        check(lib().yuf_linear_f32_planes(m, n, k, a.data_ptr(), w.data_ptr(), planes.data_ptr(), *tail))
+    elif form == "bf16":
+        check(lib().yuf_linear_bf16w(m, n, k, a.data_ptr(), w.data_ptr(), *tail))
+    else:
+        check(lib().yuf_linear_f32(m, n, k, a.data_ptr(), w.data_ptr(), *tail))
+    torch.cuda.synchronize()
+    assert torch.isnan(c[m]).all()
+    a64, w64 = a.cpu().double(), w.cpu().double()
+    z = a64 @ w64.T
+    mag = a64.abs() @ w64.abs().T
+    z = z if bias is None else z + bias.cpu().double()
+    z = (z, torch.tanh(z), torch.sigmoid(z))[act]
+    z = z if res is None else z + res.cpu().double()
+    bound = ((k + 3) * 2.0 ** -24 + (2.0 ** -16 if form == "bf16" else 0.0)) * mag + 8 * 2.0 ** -24 * (1.0 + z.abs())
+    err = (c[:m].cpu().double() - z).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())

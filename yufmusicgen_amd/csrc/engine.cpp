@@ -103,6 +103,7 @@ struct Engine {
     float *dl_buf = nullptr;         // per-XCD group activations
     int *dl_sync = nullptr;          // per-layer counter blocks, zeroed at the start of each step
     size_t dl_sync_ints = 0;         // per layer
+    int pass_rows = 0;  // rows of the running prefill chunk over all its parts (0: one part); sizes GEMM tiles
     int prefill_groups = 0;                                    // YUF_PREFILL_GROUPS=1..4: streams for the batch's parts (0: automatic)
     // The first layer's WKV-7 step launch of the last decode pass (fused
     // low-rank form), kept for yuf_engine_time_wkv_step.
@@ -381,6 +382,7 @@ GemmParams make_gemm(Engine &e, int M, int N, int K, const float *A, int lda, co
                      int ldr = 0, bool silu_pair = false) {
     GemmParams p;
     p.M = M; p.N = N; p.K = K; p.A = A; p.lda = lda; p.W = W; p.ldw = ldw; p.C = C; p.ldc = ldc;
+    p.rows = std::max(M, e.pass_rows);
     p.bias = bias; p.act = act; p.residual = residual; p.ldr = ldr; p.silu_pair = silu_pair;
     p.workspace = e.gemm_ws; p.workspace_floats = e.gemm_ws_floats;
     if (e.w_h && W >= e.w_base && W < e.w_base + e.w_floats) p.Wh = e.w_h + (W - e.w_base);
@@ -817,17 +819,20 @@ int prefill_impl(Engine &e, int n, int T, const int32_t *tokens_dev, float *logi
         // at once instead of waiting for the host to enqueue the whole pass of
         // the parts before it.
         const int layers = e.s.layers;
+        e.pass_rows = G > 1 ? n * tc : 0;
         for (int l = 0; l == 0 || l < layers; ++l) {
             const int l1 = G > 1 ? std::min(l + 1, layers) : layers;
             for (int g = 0; g < G; ++g) {
                 const int rc = forward_pass(e, acts[g], ns[g], tc, lgs[g], chunk_mode, T, t0, l, l1);
                 if (rc != YUF_OK) {
+                    e.pass_rows = 0;
                     (void)join_forked();
                     return rc;
                 }
             }
             if (l1 == layers) break;
         }
+        e.pass_rows = 0;
         ENG_TRY(join_forked(), "join");
         if (head_after) {
             const Act a0 = act_at(e, e.stream, 0, tc);

@@ -6,8 +6,8 @@
 // :107-112 (TimeMix projections), :196 (output), :306-342 (ROSA), :377 (FFN),
 // :421 (LM head).
 //
-// Kernel: 256 threads = 4 waves in a 2 x 2 arrangement; block tile 128 x 128,
-// K tile 32, double-buffered LDS.  Each wave owns a 64 x 64 sub-tile as 2 x 2
+// Kernel for K or alignments that no other takes (gemm_f32_kernel): 256 threads
+// = 4 waves in a 2 x 2 arrangement; block tile 128 x 128, K tile 32, double-buffered LDS.  Each wave owns a 64 x 64 sub-tile as 2 x 2
 // v_mfma_f32_32x32x2f32 accumulators (16 fp32 per lane each).  Operands are
 // fetched from LDS with ds_read_b128: within a K tile, lanes 0-31 contract
 // k in [0, 16) and lanes 32-63 k in [16, 32) (each MFMA sums one k of each
@@ -357,32 +357,27 @@ __device__ __forceinline__ float4 stage_read(const float *stage, int row, int c4
     return *reinterpret_cast<const float4 *>(stage + row * (WN + 4) + 4 * c4);
 }
 
-// Epilogue of the large-tile kernels: waves 4 x 2 over a 64 MI x BN tile, wave
-// (wm, wn) owns rows m0 + 16 MI wm + [0, 16 MI) and columns n0 + (BN / 2) wn +
-// [0, BN / 2), accumulator acc[i][j] the 16 x 16 block (i, j) of it (MI = 4:
-// 256-row tiles; MI = 1: 64-row tiles).  `lds` is free when it is called
-// (STAGED: wave-private staging areas of 16 x (BN / 2 + 4) floats).
-template <int BN, bool STAGED, int MI = 4>
-__device__ __forceinline__ void big_epilogue(const GemmParams &p, floatx4 (&acc)[MI][BN / 32], float *lds, int m0,
-                                             int n0, int wave, int lane) {
-    constexpr int WN = BN / 2, NT = WN / 16;
-    const int wm = wave >> 1, wn = wave & 1;
+// Epilogue of the tile kernels: the wave owns rows row0 + [0, 16 MI) and
+// columns col0 + [0, WN), accumulator acc[i][j] the 16 x 16 block (i, j) of
+// them.  `stage` is free LDS when it is called (STAGED: a wave-private staging
+// area of 16 x (WN + 4) floats).
+template <int WN, bool STAGED, int MI>
+__device__ __forceinline__ void tile_epilogue(const GemmParams &p, floatx4 (&acc)[MI][WN / 16], float *stage, int row0,
+                                              int col0, int lane) {
+    constexpr int NT = WN / 16;
     const int g4 = lane >> 4, li = lane & 15;
     // Accumulator register r of lane l: row 4 (l / 16) + r, column l % 16 of its 16 x 16 tile.
     // The parameters are read once, ahead of the LDS fences below (after a
     // fence the compiler would load each kernel-argument field again).
-    const int M = p.M, ldc = p.ldc, ldr = p.ldr, act = p.act;
+    const int M = p.M, N = p.N, ldc = p.ldc, ldr = p.ldr, act = p.act;
     float *const C = p.C;
     const float *const bias_p = p.bias, *const res_p = p.residual;
     if constexpr (STAGED) {
-        // The K loop ended with a barrier: LDS is free.  Wave-private staging areas.
         constexpr int SW = WN + 4;
-        float *stage = lds + wave * 16 * SW;
-        const int row0 = m0 + wm * 16 * MI;
         if (p.silu_pair) {
-            if constexpr (BN % 128 == 0) {
+            if constexpr (WN % 64 == 0) {
                 constexpr int HW = WN / 2;  // output columns of the wave
-                const int hcol0 = (n0 + wn * WN) / 2;
+                const int hcol0 = col0 / 2;
 #pragma unroll
                 for (int i = 0; i < MI; ++i) {
 #pragma unroll
@@ -410,7 +405,6 @@ __device__ __forceinline__ void big_epilogue(const GemmParams &p, floatx4 (&acc)
             }
             return;
         }
-        const int col0 = n0 + wn * WN;
         // One copy of the row loop per activation (a uniform branch outside it).
         auto rows = [&](auto act_c) {
             constexpr int ACT = decltype(act_c)::value;
@@ -426,7 +420,7 @@ __device__ __forceinline__ void big_epilogue(const GemmParams &p, floatx4 (&acc)
                 for (int t = 0; t < 16 * WN / 4 / 64; ++t) {
                     const int q = lane + 64 * t, row = q / (WN / 4), c4 = q % (WN / 4);
                     const int grow = row0 + i * 16 + row, col = col0 + 4 * c4;
-                    if (grow < M) {
+                    if (grow < M && col < N) {
                         float4 x = stage_read<WN>(stage, row, c4);
                         if (bias_p) {
                             const float4 b4 = *reinterpret_cast<const float4 *>(bias_p + col);
@@ -450,20 +444,20 @@ __device__ __forceinline__ void big_epilogue(const GemmParams &p, floatx4 (&acc)
         else rows(std::integral_constant<int, ACT_NONE>{});
         return;
     }
-    if constexpr (BN % 128 == 0) {
+    if constexpr (WN % 64 == 0) {
         if (p.silu_pair) {
             // Each wave's columns are whole 64-row blocks [32 "in" | 32 "gate"].
 #pragma unroll
             for (int b = 0; b < WN / 64; ++b)
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
-                    const int hcol = (n0 + wn * WN + 64 * b) / 2 + 16 * h + li;
+                    const int hcol = (col0 + 64 * b) / 2 + 16 * h + li;
                     if (hcol >= p.N / 2) continue;
 #pragma unroll
                     for (int i = 0; i < MI; ++i)
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
-                            const int row = m0 + wm * 16 * MI + i * 16 + 4 * g4 + r;
+                            const int row = row0 + i * 16 + 4 * g4 + r;
                             if (row < p.M) {
                                 const float x = acc[i][4 * b + h][r], gt = acc[i][4 * b + 2 + h][r];
                                 p.C[(size_t)row * p.ldc + hcol] = x / (1.0f + expf(-x)) * gt;
@@ -475,14 +469,14 @@ __device__ __forceinline__ void big_epilogue(const GemmParams &p, floatx4 (&acc)
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const int col = n0 + wn * WN + j * 16 + li;
+        const int col = col0 + j * 16 + li;
         if (col >= p.N) continue;
         const float bias = p.bias ? p.bias[col] : 0.0f;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm * 16 * MI + i * 16 + 4 * g4 + r;
+                const int row = row0 + i * 16 + 4 * g4 + r;
                 if (row < p.M) {
                     float x = apply_act(acc[i][j][r] + bias, p.act);
                     if (p.residual) x += p.residual[(size_t)row * p.ldr + col];
@@ -681,7 +675,8 @@ __global__ void __launch_bounds__(kBigThreads) gemm_big_kernel(GemmGroup g, int 
         lds_barrier();
     }
 
-    big_epilogue<BN, STAGED>(p, acc, lds, m0, n0, wave, lane);
+    // The K loop ended with a barrier: LDS is free.
+    tile_epilogue<WN, STAGED, 4>(p, acc, lds + wave * 16 * (WN + 4), m0 + wm * 64, n0 + wn * WN, lane);
 }
 
 // ---------------------------------------------------------------------------
@@ -832,7 +827,330 @@ __global__ void __launch_bounds__(kBigThreads) gemm_x3p_kernel(GemmGroup g, int 
         __builtin_amdgcn_s_waitcnt(kWaitVm0);
         lds_barrier();
     }
-    big_epilogue<BN, STAGED, MI>(p, acc, lds, m0, n0, wave, lane);
+    tile_epilogue<WN, STAGED, MI>(p, acc, lds + wave * 16 * (WN + 4), m0 + wm * 16 * MI, n0 + wn * WN, lane);
+}
+
+// ---------------------------------------------------------------------------
+// Small tiles with a load pipeline, for products whose 256-row tiles would
+// leave most of the 256 CUs idle (short and ragged prefills).  Such a launch is
+// bound by the latency of one tile: K / 32 steps, each of which waits out a
+// memory round trip (~0.8 us) with two LDS buffers.  Here the tile is small
+// enough for the launch to fill the chip and ST buffers keep the next k tiles
+// in flight (direct buffer -> LDS loads, counted waits).  Measured, 256-row
+// tiles -> this kernel: 333 x 640 x 640 50 -> 9 us, 333 x 640 x 2560 183 -> 26,
+// 1000 x 5120 x 640 75 -> 47, bf16 W 2200 x 1024 x 4096 199 -> 65.  What bounds
+// it now is the CU's own step (LDS reads, the split, one barrier), so a 32 x 32
+// tile, alone on its CU with one wave per SIMD, also pipelines its registers
+// (33 -> 26 us at K = 2560); for 64 x 64 and 128 x 128 tiles a second workgroup
+// on the CU hides more than that did (bf16 128 x 128: 41 us, pipelined 50).
+//
+// Blocks, swizzles, the three-part split and the per-element product order are
+// gemm_x3p_kernel's (PS_X3P: W planes; PS_X3: W fp32, split by the wave that
+// uses it) and gemm_big_kernel's bf16-weight form (PS_BF16): bit-identical to
+// them.  PS_F32 multiplies fp32 on v_mfma_f32_16x16x4f32: the arithmetic of
+// products below 256 rows (100 x 640 x 640: 62 -> 8 us; X3 took 10, its split
+// being the larger part of a lone wave's step).
+// ---------------------------------------------------------------------------
+enum PsMode : int { PS_X3P = 0, PS_X3 = 1, PS_BF16 = 2, PS_F32 = 3 };
+
+template <int MODE, int BM, int BN, int WM, int WNS, int ST, int PIPE, bool STAGED>
+__global__ void __launch_bounds__(64 * WM * WNS) gemm_ps_kernel(GemmGroup g, int per_xcd) {
+    constexpr int NW = WM * WNS, WN = BN / WNS, NT = WN / 16, MI = BM / WM / 16;
+    constexpr int AB = BM / 8;  // A blocks per k tile (8 rows x 32 k fp32 = 1 KB)
+    constexpr bool W32 = MODE == PS_X3 || MODE == PS_F32;  // W staged as fp32
+    constexpr int WBK = MODE == PS_X3P ? BN / 16 * 3 : W32 ? BN / 8 : BN / 16;  // W blocks per k tile
+    constexpr int NB = AB + WBK, PER = (NB + NW - 1) / NW, FULL = NB % NW ? NB % NW : NW;  // waves < FULL load PER blocks
+    constexpr int GM = 16;
+    static_assert(AB % NW == 0 || NW % AB == 0, "a load slot of the loop is A or W for a whole wave");
+    static_assert(ST * PER < 64, "vmcnt counts to 63");
+    static_assert(ST * NB * 1024 <= 160 * 1024 && ST * NB * 256 >= NW * 16 * (WN + 4), "LDS");
+    __shared__ __attribute__((aligned(1024))) float lds[ST * NB * 256];
+
+    const GemmParams &p = g.p[blockIdx.y];
+    const int tiles_n = g.tiles_n[blockIdx.y], total = g.total[blockIdx.y];
+    const int flat = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (flat >= total) return;
+    const int tiles_m = total / tiles_n;
+    const int grp = flat / (GM * tiles_n), rem = flat - grp * GM * tiles_n;
+    const int gm = min(GM, tiles_m - grp * GM);
+    const int bm = grp * GM + rem % gm, bn = rem / gm;
+    const int m0 = bm * BM, n0 = bn * BN;
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the LDS destination goes in M0
+    const int wm = wave / WNS, wn = wave % WNS;
+    const int g4 = lane >> 4, li = lane & 15;
+    const int lda = __builtin_amdgcn_readfirstlane(p.lda), K = __builtin_amdgcn_readfirstlane(p.K);
+    const int ldw = __builtin_amdgcn_readfirstlane(p.ldw);
+    const int KT = K / 32;
+    const int rows_a = min(BM, p.M - m0), rows_w = min(BN, p.N - n0);
+    const auto ra = make_rsrc(p.A + (size_t)m0 * lda, (uint32_t)(((size_t)(rows_a - 1) * lda + K) * 4));
+    const void *const w_base = MODE == PS_X3P ? static_cast<const void *>(p.Wp)
+                               : W32          ? static_cast<const void *>(p.W + (size_t)n0 * ldw)
+                                              : static_cast<const void *>(p.Wh + (size_t)n0 * ldw);
+    const auto rw = make_rsrc(w_base, MODE == PS_X3P ? (uint32_t)((size_t)(p.N / 16) * KT * 3 * 1024)
+                                                     : (uint32_t)(((size_t)(rows_w - 1) * ldw + K) * (W32 ? 4 : 2)));
+
+    // This lane's byte offset of each of its wave's blocks at k tile 0, and the step per k tile.
+    uint32_t off[PER];
+    const int ar = lane >> 3, apos = lane & 7, hr = lane >> 2, hpos = lane & 3;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int b = wave + NW * i;
+        if (b < AB) {
+            off[i] = (uint32_t)(((b * 8 + ar) * lda + 4 * (apos ^ ar ^ (b & 1))) * 4);
+        } else {
+            const int bb = b - AB;
+            if constexpr (MODE == PS_X3P)
+                off[i] = (uint32_t)((((bn * (BN / 16) + bb / 3) * KT) * 3 + bb % 3) * 1024 + lane * 16);
+            else if constexpr (W32)
+                off[i] = (uint32_t)(((bb * 8 + ar) * ldw + 4 * (apos ^ ar ^ (bb & 1))) * 4);
+            else
+                off[i] = (uint32_t)(((bb * 16 + hr) * ldw + 8 * (hpos ^ x3p_swz(hr))) * 2);
+        }
+    }
+    constexpr int kWStep = MODE == PS_X3P ? 3072 : W32 ? 128 : 64;
+    auto issue = [&](int kt, int buf) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int b = wave + NW * i;
+            if (i == PER - 1 && FULL != NW && wave >= FULL) break;
+            lds_void_t *dst = (lds_void_t *)(lds + (buf * NB + b) * 256);
+            const uint32_t o = off[i];
+            if (NW * i + NW <= AB || b < AB)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, o, kt * 128, 0, 0);
+            else
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, dst, 16, o, kt * kWStep, 0, 0);
+        }
+    };
+
+    floatx4 acc[MI][NT];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int fa = (li & 7) ^ (li >> 3);
+    const int fo = (li >> 3) * 256 + (li & 7) * 32;  // fp32 fragment: row li of two 8-row blocks
+    const int o0 = fo + ((2 * g4) ^ fa) * 4, o1 = fo + ((2 * g4 + 1) ^ fa) * 4;
+    const int oh = li * 32 + ((g4 ^ x3p_swz(li)) * 8);  // bf16 fragment
+
+    // A wave's fragments of a k tile: fp32 as read from LDS, then split.
+    constexpr int AP = MODE == PS_BF16 ? 2 : 3, WP = MODE == PS_BF16 ? 1 : 3;
+    struct Raw {
+        floatx4 a[MI][2], w[W32 ? NT : 1][2];
+    };
+    struct Parts {
+        bf16x8 a[AP][MI], w[WP][NT];
+    };
+    auto read_raw = [&](Raw &f, int buf) {
+        const float *base = lds + buf * NB * 256, *ab = base + wm * 2 * MI * 256, *wb = base + AB * 256;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            f.a[i][0] = *reinterpret_cast<const floatx4 *>(ab + i * 512 + o0);
+            f.a[i][1] = *reinterpret_cast<const floatx4 *>(ab + i * 512 + o1);
+        }
+        if constexpr (W32) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                f.w[j][0] = *reinterpret_cast<const floatx4 *>(wb + (WNS * j + wn) * 512 + o0);
+                f.w[j][1] = *reinterpret_cast<const floatx4 *>(wb + (WNS * j + wn) * 512 + o1);
+            }
+        }
+    };
+    auto read_w = [&](Parts &f, int buf) {  // W parts that are ready in LDS
+        if constexpr (!W32) {
+            const __bf16 *bh = reinterpret_cast<const __bf16 *>(lds + (buf * NB + AB) * 256);
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < WP; ++q)
+                    f.w[q][j] = *reinterpret_cast<const bf16x8 *>(bh + ((WNS * j + wn) * WP + q) * 512 + oh);
+        }
+    };
+    auto split = [&](const Raw &x, Parts &f) {
+        if constexpr (MODE == PS_F32) return;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            if constexpr (MODE == PS_BF16) split_bf16x8(x.a[i][0], x.a[i][1], f.a[0][i], f.a[1][i]);
+            else split3_x8(x.a[i][0], x.a[i][1], f.a[0][i], f.a[1][i], f.a[AP - 1][i]);
+        }
+        if constexpr (MODE == PS_X3) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j) split3_x8(x.w[j][0], x.w[j][1], f.w[0][j], f.w[1][j], f.w[WP - 1][j]);
+        }
+    };
+    // Part products in the fixed order (a3 w1, a1 w3, a2 w2, a2 w1, a1 w2, a1 w1, or
+    // hi then lo), all accumulators of the wave per part product: independent
+    // MFMAs follow each other.
+    constexpr int NP = MODE == PS_BF16 ? 2 : 6;
+    auto products = [&](const Raw &x, const Parts &f) {
+        if constexpr (MODE == PS_F32) {  // k step r of half h: k = 8 g4 + 4 h + r of the tile, both operands
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int i = 0; i < MI; ++i)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[i][h][r], x.w[j][h][r], acc[i][j], 0, 0, 0);
+            return;
+        }
+        constexpr int pa[6] = {MODE == PS_BF16 ? 0 : 2, MODE == PS_BF16 ? 1 : 0, 1, 1, 0, 0};
+        constexpr int pw[6] = {0, MODE == PS_BF16 ? 0 : 2, 1, 0, 1, 0};
+#pragma unroll
+        for (int q = 0; q < NP; ++q)
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.a[pa[q]][i], f.w[pw[q]][j], acc[i][j], 0, 0, 0);
+    };
+
+#pragma unroll
+    for (int t = 0; t < ST - 1 + PIPE; ++t)
+        if (t < KT) issue(t, t);
+    // Wait for all but the newest `tiles` k tiles of this wave's loads (`all`:
+    // for all of them) and for its LDS reads, then meet the other waves.  One
+    // asm block: around the barrier builtin the compiler waits for every
+    // outstanding load into LDS, which empties the pipeline.
+    auto arrive = [&](bool all, auto tiles) {
+        constexpr int n = decltype(tiles)::value;
+        if (all) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        else if (FULL == NW || wave < FULL) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n * PER) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(n * (PER - 1)) : "memory");
+    };
+    int buf = 0;  // tile kt's buffer
+    if constexpr (PIPE) {
+        // One wave per SIMD: the LDS latency, the split's VALU chain and the
+        // dependent MFMA chain of a tile run in different steps.  Step kt
+        // multiplies tile kt while it splits tile kt + 1's fp32 fragments, reads
+        // tile kt + 2's from LDS and loads tile kt + ST into the buffer that
+        // tile kt has left.
+        arrive(KT < ST, std::integral_constant<int, ST - 2>{});
+        Raw x0, x1;
+        Parts f0, f1;
+        read_raw(x0, 0);
+        read_w(f0, 0);
+        if (KT > 1) read_raw(x1, 1);
+        split(x0, f0);
+        // cur: tile kt's parts; xn: tile kt + 1's raw fragments; xf: free, takes tile kt + 2's.
+        auto step = [&](int kt, const Parts &cur, Parts &nxt, Raw &xf, const Raw &xn) {
+            const int b1 = buf == ST - 1 ? 0 : buf + 1, b2 = b1 == ST - 1 ? 0 : b1 + 1;
+            // Tile kt + 2 is in LDS for every wave, and every wave has read tile kt.
+            arrive(kt + ST > KT, std::integral_constant<int, ST - 3>{});
+            if (kt + ST < KT) issue(kt + ST, buf);
+            if constexpr (MODE == PS_F32) products(xf, cur);
+            read_raw(xf, b2);  // past the last tile: LDS that is allocated, values unused
+            read_w(nxt, b1);
+            split(xn, nxt);
+            if constexpr (MODE != PS_F32) products(xn, cur);
+            buf = b1;
+        };
+        int kt = 0;
+        for (; kt + 1 < KT; kt += 2) {
+            step(kt, f0, f1, x0, x1);
+            step(kt + 1, f1, f0, x1, x0);
+        }
+        if (kt < KT) products(x0, f0);
+    } else {
+        for (int kt = 0; kt < KT; ++kt) {
+            // Tile kt is in LDS for every wave, and every wave has read tile kt - 1.
+            arrive(kt + ST - 1 > KT, std::integral_constant<int, ST - 2>{});
+            if (kt + ST - 1 < KT) issue(kt + ST - 1, buf == 0 ? ST - 1 : buf - 1);
+            Raw x;
+            Parts f;
+            read_raw(x, buf);
+            read_w(f, buf);
+            split(x, f);
+            products(x, f);
+            buf = buf == ST - 1 ? 0 : buf + 1;
+        }
+    }
+
+    // Epilogue: block (i, j) of the wave is rows m0 + 16 (wm MI + i), columns
+    // n0 + 16 (WNS j + wn).  A SiLU group of 64 columns (two in blocks, two gate
+    // blocks) is G = 2 / WNS in blocks, then their G gate blocks, of each wave.
+    const int row0 = m0 + wm * 16 * MI;
+    constexpr int G = WNS <= 2 ? 2 / WNS : 1;
+    constexpr bool PAIRS = BN % 64 == 0 && WNS <= 2;
+    auto silu_col = [&](int t) { return n0 / 2 + 32 * (t / G) + 16 * (WNS == 2 ? wn : t % G); };  // wave's output block t
+    if constexpr (!STAGED) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int col = n0 + 16 * (WNS * j + wn) + li;
+            if (p.silu_pair && (!PAIRS || j % (2 * G) >= G)) continue;
+            const int ccol = p.silu_pair ? silu_col(j / (2 * G) * G + j % G) + li : col;
+            if (col >= p.N) continue;
+            const float bias = p.bias ? p.bias[col] : 0.0f;
+#pragma unroll
+            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int row = row0 + i * 16 + 4 * g4 + r;
+                    if (row >= p.M) continue;
+                    float x = acc[i][j][r];
+                    if (p.silu_pair) {
+                        x = x / (1.0f + expf(-x)) * acc[i][j + G < NT ? j + G : j][r];
+                    } else {
+                        x = apply_act(x + bias, p.act);
+                        if (p.residual) x += p.residual[(size_t)row * p.ldr + col];
+                    }
+                    p.C[(size_t)row * p.ldc + ccol] = x;
+                }
+        }
+    } else {
+        // Through wave-private LDS, so C, residual and bias move as 16-byte runs.
+        const int M = p.M, N = p.N, ldc = p.ldc, ldr = p.ldr, act = p.act;
+        const bool silu = p.silu_pair;
+        float *const C = p.C;
+        const float *const bias_p = p.bias, *const res_p = p.residual;
+        constexpr int SW = WN + 4;
+        float *stage = lds + wave * 16 * SW;
+        lds_barrier();  // every wave has read its last tile
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+            if (silu) {
+                if constexpr (PAIRS) {
+#pragma unroll
+                    for (int t = 0; t < NT / 2; ++t)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const int j = t / G * 2 * G + t % G;
+                            const float x = acc[i][j][r];
+                            stage[(4 * g4 + r) * SW + 16 * t + li] = x / (1.0f + expf(-x)) * acc[i][j + G][r];
+                        }
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) stage[(4 * g4 + r) * SW + 16 * j + li] = acc[i][j][r];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+            // Four lanes per 16-column block row; SiLU: half the blocks.
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const int row = lane >> 2, c4 = (lane & 3) * 4, grow = row0 + i * 16 + row;
+                const int col = n0 + 16 * (WNS * t + wn) + c4;
+                if (silu) {
+                    if (PAIRS && 2 * t < NT && grow < M)
+                        *reinterpret_cast<floatx4 *>(C + (size_t)grow * ldc + silu_col(t) + c4) =
+                            *reinterpret_cast<const floatx4 *>(stage + row * SW + 16 * t + c4);
+                } else if (grow < M && col < N) {
+                    floatx4 x = *reinterpret_cast<const floatx4 *>(stage + row * SW + 16 * t + c4);
+                    if (bias_p) x += *reinterpret_cast<const floatx4 *>(bias_p + col);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) x[q] = apply_act(x[q], act);
+                    if (res_p) x += *reinterpret_cast<const floatx4 *>(res_p + (size_t)grow * ldr + col);
+                    *reinterpret_cast<floatx4 *>(C + (size_t)grow * ldc + col) = x;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        }
+    }
 }
 
 // fp32 W [N][ldw] -> X3 planes (layout above): one thread per 8 consecutive k of a row.
@@ -1672,6 +1990,122 @@ bool use_x3(const GemmGroup &g, int n) {
     return true;
 }
 
+// A tile shape and the measured time (us) of one 32-k step of it: of tiles that
+// have their CUs to themselves, and of each full round of 256 tiles.
+struct TileCost {
+    int id, bm, bn;
+    float alone, round;
+};
+// gemm_ps_kernel's tiles per mode.
+constexpr TileCost kPsTiles[4][4] = {
+    {{1, 32, 32, 0.30f, 0.168f}, {2, 64, 64, 0.60f, 0.45f}, {3, 128, 128, 1.22f, 1.25f}, {}},                        // PS_X3P
+    {{1, 32, 32, 0.35f, 0.20f}, {2, 64, 64, 0.70f, 0.48f}, {3, 128, 128, 1.65f, 1.65f}, {}},                         // PS_X3
+    {{1, 32, 32, 0.23f, 0.10f}, {2, 64, 64, 0.32f, 0.205f}, {3, 128, 128, 0.64f, 0.65f}, {4, 64, 128, 0.47f, 0.34f}},  // PS_BF16
+    {{1, 32, 32, 0.24f, 0.195f}, {2, 64, 64, 0.67f, 0.55f}, {5, 32, 64, 0.40f, 0.33f}, {}},                          // PS_F32
+};
+// The 256-row tiles of the same forms (64-wide X3P: 64-row tiles), widths 256, 160, 128, 64.
+constexpr TileCost kBigTiles[3][4] = {
+    {{0, 256, 256, 3.55f, 4.65f}, {0, 256, 160, 2.4f, 3.0f}, {0, 256, 128, 2.05f, 2.6f}, {0, 64, 64, 0.53f, 0.9f}},
+    {{0, 256, 256, 4.1f, 5.4f}, {0, 256, 160, 2.8f, 3.5f}, {0, 256, 128, 2.3f, 2.9f}, {0, 256, 64, 1.9f, 2.2f}},
+    {{0, 256, 256, 1.6f, 1.95f}, {0, 256, 160, 1.2f, 1.7f}, {0, 256, 128, 1.05f, 1.6f}, {0, 256, 64, 0.87f, 1.5f}},
+};
+
+template <int MODE, bool STAGED>
+void launch_ps_tile(const GemmGroup &g, int id, int per_xcd, dim3 grid, hipStream_t stream) {
+    const dim3 b4(256), b8(512);
+    if (id == 1) {
+        hipLaunchKernelGGL((gemm_ps_kernel<MODE, 32, 32, 2, 2, 5, 1, STAGED>), grid, b4, 0, stream, g, per_xcd);
+    } else if (id == 2) {
+        if constexpr (MODE == PS_BF16)
+            hipLaunchKernelGGL((gemm_ps_kernel<MODE, 64, 64, 4, 1, 4, 0, STAGED>), grid, b4, 0, stream, g, per_xcd);
+        else
+            hipLaunchKernelGGL((gemm_ps_kernel<MODE, 64, 64, 2, 2, 3, 0, STAGED>), grid, b4, 0, stream, g, per_xcd);
+    } else if (id == 3) {
+        if constexpr (MODE != PS_F32)
+            hipLaunchKernelGGL((gemm_ps_kernel<MODE, 128, 128, 4, 2, 2, 0, STAGED>), grid, b8, 0, stream, g, per_xcd);
+    } else if (id == 4) {
+        if constexpr (MODE == PS_BF16)
+            hipLaunchKernelGGL((gemm_ps_kernel<MODE, 64, 128, 2, 2, 3, 0, STAGED>), grid, b4, 0, stream, g, per_xcd);
+    } else {
+        if constexpr (MODE == PS_F32)
+            hipLaunchKernelGGL((gemm_ps_kernel<MODE, 32, 64, 2, 2, 5, 1, STAGED>), grid, b4, 0, stream, g, per_xcd);
+    }
+}
+
+hipError_t launch_ps(GemmGroup &g, int n, int mode, const TileCost &t, hipStream_t stream) {
+    int most = 0;
+    bool staged = true;  // 16-byte epilogue accesses need aligned C / residual / bias rows
+    for (int i = 0; i < n; ++i) {
+        const GemmParams &p = g.p[i];
+        g.tiles_n[i] = (p.N + t.bn - 1) / t.bn;
+        g.total[i] = ((p.M + t.bm - 1) / t.bm) * g.tiles_n[i];
+        most = std::max(most, g.total[i]);
+        const uintptr_t bits = reinterpret_cast<uintptr_t>(p.C) | reinterpret_cast<uintptr_t>(p.residual) |
+                               reinterpret_cast<uintptr_t>(p.bias);
+        staged = staged && (bits & 15) == 0 && p.N % 4 == 0 && p.ldc % 4 == 0 && (!p.residual || p.ldr % 4 == 0);
+    }
+    const int per_xcd = (most + kXcds - 1) / kXcds;
+    const dim3 grid(per_xcd * kXcds, n);
+    auto go = [&](auto m) {
+        constexpr int MODE = decltype(m)::value;
+        if (staged) launch_ps_tile<MODE, true>(g, t.id, per_xcd, grid, stream);
+        else launch_ps_tile<MODE, false>(g, t.id, per_xcd, grid, stream);
+    };
+    if (mode == PS_X3P) go(std::integral_constant<int, PS_X3P>{});
+    else if (mode == PS_X3) go(std::integral_constant<int, PS_X3>{});
+    else if (mode == PS_BF16) go(std::integral_constant<int, PS_BF16>{});
+    else go(std::integral_constant<int, PS_F32>{});
+    return hipGetLastError();
+}
+
+// The tile of gemm_ps_kernel a group takes, or nullptr: it takes the 256-row
+// tiles of width big_bn (0: it has none and falls back to another kernel).
+// The estimate of a launch is its rounds of 256 tiles times the measured time
+// of a k step; tiles are counted over the rows of the whole call, since a
+// prefill's parts run side by side.  (X3P, us, this kernel against the 256-row
+// tiles: 333 x 640 x 640 9 / 50, 333 x 640 x 2560 26 / 183, 1000 x 5120 x 640 45 / 76,
+// 4096 x 5120 x 640 131 / 164; 16384 x 5120 x 640 503 / 468 keeps the latter.)
+// X3P products with K <= 128 move to it below 2048 rows only: there the output
+// write bounds both (640 x 128: 6.3 / 8.1 at 1000 rows, 11 / 9.8 at 4096).
+const TileCost *ps_tile(const GemmGroup &g, int n, int mode, int big_bn) {
+    bool silu = false, n128 = true;
+    int K = 0, rows = 0;
+    for (int i = 0; i < n; ++i) {
+        const GemmParams &p = g.p[i];
+        const void *w = mode == PS_BF16 ? (const void *)p.Wh : (const void *)p.W;
+        if (p.K % 32 != 0 || p.lda % 4 != 0 || (reinterpret_cast<uintptr_t>(p.A) & 15) != 0) return nullptr;
+        if (mode == PS_X3P ? p.N % 64 != 0
+                           : (p.ldw % (mode == PS_BF16 ? 8 : 4) != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0))
+            return nullptr;
+        silu = silu || p.silu_pair;
+        n128 = n128 && p.N % 128 == 0;
+        K = std::max(K, p.K);
+        rows = std::max(rows, std::max(p.rows, p.M));
+    }
+    if (mode == PS_X3P && K <= 128 && rows >= 2048 && big_bn) return nullptr;
+    const auto cost = [&](const TileCost &t) {
+        long long tiles = 0;
+        for (int i = 0; i < n; ++i)
+            tiles += (long long)((std::max(g.p[i].rows, g.p[i].M) + t.bm - 1) / t.bm) * ((g.p[i].N + t.bn - 1) / t.bn);
+        if (tiles <= 256) return t.alone >= t.round ? t.alone : t.alone + (t.round - t.alone) * (float)tiles / 256.0f;
+        return std::max(t.alone, t.round * (float)((tiles + 255) / 256));
+    };
+    const TileCost *best = nullptr;
+    float least = 0.0f;
+    if (big_bn && mode != PS_F32)
+        for (const TileCost &t : kBigTiles[mode])
+            if (t.bn == big_bn) least = cost(t);
+    for (const TileCost &t : kPsTiles[mode]) {
+        if (!t.id || (silu && t.bn < 64) || (t.bn == 128 && !n128)) continue;
+        const float c = cost(t);
+        if (least == 0.0f || c < least) {
+            least = c;
+            best = &t;
+        }
+    }
+    return best;
+}
+
 template <int NT, int MI, int PRO, bool WB, int S>
 void launch_dec_s(const DecodeGroup &g, dim3 grid, hipStream_t stream) {
     if constexpr (S <= dec_cap(NT, MI, PRO, WB)) {
@@ -1912,6 +2346,13 @@ hipError_t launch_gemm_group(const GemmParams *ps, int count, hipStream_t stream
         }
         if (nh > 0) {
             if (!(f256 || f160 || f128 || f64)) return hipErrorInvalidValue;
+            if (const TileCost *t = ps_tile(gh, nh, PS_BF16, f256 ? 256 : f160 ? 160 : f128 ? 128 : 64)) {
+                const hipError_t e = launch_ps(gh, nh, PS_BF16, *t, stream);
+                if (e != hipSuccess) return e;
+                nh = 0;
+            }
+        }
+        if (nh > 0) {
             const int bn = f256 ? 256 : f160 ? 160 : f128 ? 128 : 64;
             bool staged = true;
             for (int i = 0; i < nh; ++i) {
@@ -1969,6 +2410,10 @@ hipError_t launch_gemm_group(const GemmParams *ps, int count, hipStream_t stream
     }
     if (fit256 || fit160 || fit128 || fit64) {
         const int bn = fit256 ? 256 : fit160 ? 160 : fit128 ? 128 : 64;
+        if (use_x3(g, n)) {
+            const int mode = use_x3p(g, n) ? PS_X3P : PS_X3;
+            if (const TileCost *t = ps_tile(g, n, mode, bn)) return launch_ps(g, n, mode, *t, stream);
+        }
         int big_max = 0;
         for (int i = 0; i < n; ++i) {
             g.tiles_n[i] = g.p[i].N / bn;
@@ -2035,6 +2480,8 @@ hipError_t launch_gemm_group(const GemmParams *ps, int count, hipStream_t stream
         }
         return hipGetLastError();
     }
+    // Fewer than 256 rows, or columns that no large tile fits: fp32 MFMA.
+    if (const TileCost *t = ps_tile(g, n, PS_F32, 0)) return launch_ps(g, n, PS_F32, *t, stream);
     const int per_xcd = (max_total + kXcds - 1) / kXcds;
     hipLaunchKernelGGL(gemm_f32_kernel, dim3(per_xcd * kXcds, n), dim3(kThreads), 0, stream, g, per_xcd);
     return hipGetLastError();

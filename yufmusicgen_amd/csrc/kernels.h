@@ -87,6 +87,9 @@ hipError_t launch_rosa_segmented(const RosaParams &p, const float *AL, int L, fl
 enum GemmAct : int { ACT_NONE = 0, ACT_TANH = 1, ACT_SIGMOID = 2 };
 struct GemmParams {
     int M = 0, N = 0, K = 0;
+    // Rows of the whole call when these M are one of several parts that run
+    // side by side (0: M); only the choice of tile sizes reads it.
+    int rows = 0;
     const float *A = nullptr;
     int lda = 0;
     const float *W = nullptr;
