@@ -192,8 +192,8 @@ def bench_wkv_step(iters: int) -> dict:
 
 def bench_rosa(iters: int) -> dict:
     """ROSA scan of one C3 layer (B=8, T=2048, D=128, gated read) through the
-    operator entry point (segmented form: A^64 on the device, segments from
-    zero, carry chain, segments again): 4 (4 B T D + 2 B D) bytes = 33.6 MB."""
+    operator entry point (segmented form: A^128 on the device, segments from
+    zero, then the carry and the segments again): 4 (4 B T D + 2 B D) bytes = 33.6 MB."""
     import torch
 
     from yufmusicgen_amd._lib import check, lib
@@ -214,7 +214,7 @@ def bench_rosa(iters: int) -> dict:
     achieved = nbytes / (ms * 1e-3) / 1e9
     return {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "kernel": "rosa operator, segmented (rosa_power/scan/carry/scan; C3 layer: B=8 T=2048 D=128)",
+            "kernel": "rosa operator, segmented (rosa_seg_kernel twice; C3 layer: B=8 T=2048 D=128)",
             "algorithmic_bytes": nbytes, "avg_us": round(ms * 1e3, 2)}
 
 

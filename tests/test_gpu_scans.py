@@ -214,3 +214,29 @@ def test_rosa_chunked_continuation():
         outs.append(r)
     torch.testing.assert_close(torch.cat(outs, dim=1), full, rtol=RTOL, atol=ATOL)
     torch.testing.assert_close(m, m_full, rtol=RTOL, atol=ATOL)
+
+
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("steps", [2, 31, 33, 192, 193, 320, 641, 1111, 4161])
+def test_rosa_segments(dim, steps):
+    """The segment kernel at the edges of its 32-token chunks and of its segment
+    rule (one segment up to 192 tokens, 64- then 128-token segments with a ragged
+    last one, the separate carry pass above 32 segments), gated and not, against
+    the float64 oracle, with the memory updated in place."""
+    from yufmusicgen_amd._lib import check, lib
+
+    print(f"rosa segments D={dim} T={steps}", flush=True)
+    batch = 2
+    cand, write, read_raw, decay, u = (_dev(x) for x in rosa_inputs(31 + dim, batch, steps, dim))
+    m0 = np.random.default_rng(8).standard_normal((batch, dim)).astype(np.float32)
+    t64 = [x.cpu().double() for x in (cand, write, read_raw, decay, u)] + [torch.from_numpy(m0).double()]
+    for gated in (True, False):
+        mem, out = _dev(m0), torch.full((batch, steps, dim), float("nan"), device="cuda")
+        check(lib().yuf_rosa_scan_f32(batch, steps, dim, cand.data_ptr(), write.data_ptr(),
+                                      read_raw.data_ptr() if gated else None, decay.data_ptr(), u.data_ptr(),
+                                      mem.data_ptr(), mem.data_ptr(), out.data_ptr(),
+                                      torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        re, me = orosa.rosa_scan(*t64, gated=gated)
+        np.testing.assert_allclose(out.cpu().numpy(), re.numpy(), rtol=RTOL, atol=ATOL)
+        np.testing.assert_allclose(mem.cpu().numpy(), me.numpy(), rtol=RTOL, atol=ATOL)

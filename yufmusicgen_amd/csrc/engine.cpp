@@ -43,12 +43,10 @@ struct LayerW {
     const float *ln_o_w, *ln_o_b, *ln_r_w, *ln_r_b;
     const float *rosa_w3, *rosa_b3, *rosa_hh, *rosa_decay, *rosa_out;
     const float *ln_f_w, *ln_f_b, *ffn_cat, *ffn_out;
-    const float *rosa_al;  // A^kRosaSeg of the ROSA transition, [D][D] row-major
+    const float *rosa_al[2];  // A^64 and A^128 of the ROSA transition, [D][D] row-major (D in {64, 128, 256})
     const float *rosa_u, *rosa_lam;  // u = normalize(householder), lambda = sigmoid(decay), [D]
 };
 
-// Segment length of the segmented ROSA prefill scan.
-constexpr int kRosaSeg = 64;
 constexpr int kFfnParts = 4;  // K split of the decode FFN output product (partials summed by their consumer)
 
 struct DeviceBuf {
@@ -91,7 +89,8 @@ struct Engine {
     float *h = nullptr, *xn = nullptr, *mix = nullptr, *r = nullptr, *k = nullptr, *v = nullptr, *wr = nullptr,
           *al = nullptr, *g = nullptr, *lr = nullptr, *y = nullptr, *z = nullptr, *rosa3 = nullptr, *rread = nullptr,
           *ffn = nullptr, *hl = nullptr;
-    float *rz = nullptr, *rcarry = nullptr;  // segmented ROSA scratch
+    float *rz = nullptr;  // segmented ROSA scratch: 2 rows of D floats per segment
+    DeviceBuf rosa_al;
     float *kpart = nullptr;  // [kFfnParts][max_streams][d]: K-split partials of the decode FFN output
     bool rosa_segmented = true;                                // YUF_ROSA_SEGMENTED=0 disables
     bool decode_fusion = true;                                 // YUF_DECODE_FUSION=0: separate low-rank GEMM and ROSA step
@@ -301,14 +300,12 @@ int build_weights(const Checkpoint &ck, std::vector<float> &host, std::vector<si
         }
         if (!mat("ffn_out.weight", d, hid)) return YUF_ERR_FORMAT;
         {
-            // A^L for the segmented ROSA scan, A = diag(lambda) (I - 2 u u^T) with
             // lambda = sigmoid(decay), u = householder / max(|householder|, 1e-12)
-            // (yufmusicgen/model.py:300-301): column j is A applied L times to e_j,
-            // in double precision through the rank-one form A x = lambda (x - 2 (u.x) u).
+            // (yufmusicgen/model.py:300-301).
             const float *hh = get(pre + "rosa.householder", {D});
             const float *dec = get(pre + "rosa.decay", {D});
             if (!hh || !dec) return YUF_ERR_FORMAT;
-            std::vector<double> u((size_t)D), lam((size_t)D), x((size_t)D);
+            std::vector<double> u((size_t)D), lam((size_t)D);
             double nrm = 0.0;
             for (long long j = 0; j < D; ++j) nrm += (double)hh[j] * hh[j];
             nrm = std::max(std::sqrt(nrm), 1e-12);
@@ -316,18 +313,6 @@ int build_weights(const Checkpoint &ck, std::vector<float> &host, std::vector<si
                 u[(size_t)j] = hh[j] / nrm;
                 lam[(size_t)j] = 1.0 / (1.0 + std::exp(-(double)dec[j]));
             }
-            std::vector<float> al((size_t)(D * D));
-            for (long long j = 0; j < D; ++j) {
-                std::fill(x.begin(), x.end(), 0.0);
-                x[(size_t)j] = 1.0;
-                for (int step = 0; step < kRosaSeg; ++step) {
-                    double pr = 0.0;
-                    for (long long i = 0; i < D; ++i) pr += u[(size_t)i] * x[(size_t)i];
-                    for (long long i = 0; i < D; ++i) x[(size_t)i] = lam[(size_t)i] * (x[(size_t)i] - 2.0 * pr * u[(size_t)i]);
-                }
-                for (long long i = 0; i < D; ++i) al[(size_t)(i * D + j)] = (float)x[(size_t)i];
-            }
-            append(al.data(), al.size());
             std::vector<float> uf((size_t)D), lf((size_t)D);
             for (long long j = 0; j < D; ++j) {
                 uf[(size_t)j] = (float)u[(size_t)j];
@@ -439,7 +424,7 @@ int gemm_group(hipStream_t st, const GemmParams *ps, int count) {
 struct Act {
     hipStream_t st = nullptr;
     float *h, *xn, *mix, *r, *k, *v, *wr, *al, *g, *lr, *y, *z, *rosa3, *rread, *ffn, *hl;
-    float *rz, *rcarry;  // segmented ROSA scratch (segment rows of kRosaSeg tokens)
+    float *rz;  // segmented ROSA scratch of these streams
     const int *tokens, *slots;
     int *bad;     // out-of-range token flag the embedding sets
     int *rcount;  // fused ROSA-out tile counters of this group of streams
@@ -461,8 +446,7 @@ Act act_at(Engine &e, hipStream_t st, int s0, int Tc) {
     a.rosa3 = e.rosa3 + m0 * 3 * s.rosa; a.rread = e.rread + m0 * s.rosa;
     a.ffn = e.ffn + m0 * 4 * d;
     a.hl = e.hl + (size_t)s0 * d;
-    const size_t seg0 = (m0 / kRosaSeg) * s.rosa;
-    a.rz = e.rz + seg0; a.rcarry = e.rcarry + seg0;
+    a.rz = e.rz + rosa_seg_scratch(s0, Tc, s.rosa);
     a.tokens = e.tokens_dev + m0;
     a.slots = e.slots_dev + s0;
     a.bad = e.bad_dev;
@@ -659,19 +643,20 @@ int forward_pass(Engine &e, const Act &a, int n, int Tc, float *logits, int mode
         } else {
             RosaParams rp;
             rp.B = n; rp.T = Tc; rp.D = D; rp.ld = 3 * D;
-            if (Tc == 1) {
-                // The single-token kernel applies the gates itself.
-                rp.cand = a.rosa3; rp.write = a.rosa3 + D; rp.read_raw = a.rosa3 + 2 * D;
-            } else {
-                // Gates on all M rows in parallel, so the sequential scan only loads e and the gate.
-                ENG_TRY(launch_rosa_gates(a.rosa3, M, D, 3 * D, st), "rosa_gates");
-                rp.e_pre = a.rosa3; rp.g_pre = a.rosa3 + D;
-            }
-            rp.decay = w.rosa_decay; rp.direction = w.rosa_hh; rp.raw_params = true;
             rp.memory_in = ros; rp.memory_out = ros; rp.slot = a.slots; rp.read_out = a.rread;
-            if (e.rosa_segmented && Tc > 1 && rosa_segmented_ok(Tc, D, kRosaSeg)) {
-                ENG_TRY(launch_rosa_segmented(rp, w.rosa_al, kRosaSeg, a.rz, a.rcarry, st), "rosa segmented");
+            rp.cand = a.rosa3; rp.write = a.rosa3 + D; rp.read_raw = a.rosa3 + 2 * D;
+            if (e.rosa_segmented && rosa_seg_ok(Tc, D)) {
+                // The segment kernel applies the gates itself.
+                rp.decay = w.rosa_lam; rp.direction = w.rosa_u;
+                ENG_TRY(launch_rosa_segmented(rp, w.rosa_al[rosa_seg_len(Tc) == 64 ? 0 : 1], a.rz, st), "rosa segmented");
             } else {
+                if (Tc > 1) {
+                    // Gates on all M rows in parallel, so the sequential scan only loads e and the
+                    // gate (the single-token kernel applies them itself).
+                    ENG_TRY(launch_rosa_gates(a.rosa3, M, D, 3 * D, st), "rosa_gates");
+                    rp.e_pre = a.rosa3; rp.g_pre = a.rosa3 + D;
+                }
+                rp.decay = w.rosa_decay; rp.direction = w.rosa_hh; rp.raw_params = true;
                 ENG_TRY(launch_rosa(rp, st), "rosa");
             }
             if ((rc = gemm(e, st, M, d, D, a.rread, D, w.rosa_out, D, a.h, d, nullptr, ACT_NONE, a.h, d)) != YUF_OK)
@@ -1075,8 +1060,17 @@ extern "C" int yuf_engine_create_ex(const yuf_ckpt *ckpt, int max_streams, int m
         w.ln_o_w = nxt(); w.ln_o_b = nxt(); w.ln_r_w = nxt(); w.ln_r_b = nxt();
         w.rosa_w3 = nxt(); w.rosa_b3 = nxt(); w.rosa_hh = nxt(); w.rosa_decay = nxt(); w.rosa_out = nxt();
         w.ln_f_w = nxt(); w.ln_f_b = nxt(); w.ffn_cat = nxt(); w.ffn_out = nxt();
-        w.rosa_al = nxt();
         w.rosa_u = nxt(); w.rosa_lam = nxt();
+    }
+    if (rosa_seg_ok(2, s.rosa)) {
+        const size_t dd = (size_t)s.rosa * s.rosa;
+        ENG_TRY(hipMalloc(&e.rosa_al.p, 2 * dd * s.layers * sizeof(float)), "rosa powers alloc");
+        float *al = static_cast<float *>(e.rosa_al.p);
+        for (LayerW &w : e.layers)
+            for (int i = 0; i < 2; ++i, al += dd) {
+                ENG_TRY(launch_rosa_power(s.rosa, 64 << i, w.rosa_lam, w.rosa_u, al, e.stream), "rosa powers");
+                w.rosa_al[i] = al;
+            }
     }
     {
         // Tiled copies of the decode products' matrices (from the host image).
@@ -1178,7 +1172,7 @@ extern "C" int yuf_engine_create_ex(const yuf_ckpt *ckpt, int max_streams, int m
     e.gemm_ws_floats = ws;
     const size_t sizes[] = {Mx * d, Mx * d, 6 * Mx * d, Mx * d, Mx * d, Mx * d, Mx * d, Mx * d, Mx * d,
                             3 * Mx * s.low_rank, Mx * d, Mx * d, Mx * 3 * s.rosa, Mx * s.rosa, Mx * 4 * d,
-                            (size_t)max_streams * d, ws, Mx / kRosaSeg * s.rosa + s.rosa, Mx / kRosaSeg * s.rosa + s.rosa,
+                            (size_t)max_streams * d, ws, 2 * (Mx / 64 + max_streams) * s.rosa + 80 * (size_t)max_streams,
                             (size_t)kFfnParts * max_streams * d};
     size_t total = 0;
     for (size_t z : sizes) total += ((z * sizeof(float) + 255) / 256) * 256;
@@ -1186,7 +1180,7 @@ extern "C" int yuf_engine_create_ex(const yuf_ckpt *ckpt, int max_streams, int m
     {
         char *cur = static_cast<char *>(e.work.p);
         float **dst[] = {&e.h, &e.xn, &e.mix, &e.r, &e.k, &e.v, &e.wr, &e.al, &e.g, &e.lr, &e.y, &e.z, &e.rosa3,
-                         &e.rread, &e.ffn, &e.hl, &e.gemm_ws, &e.rz, &e.rcarry, &e.kpart};
+                         &e.rread, &e.ffn, &e.hl, &e.gemm_ws, &e.rz, &e.kpart};
         for (size_t i = 0; i < sizeof(sizes) / sizeof(sizes[0]); ++i) *dst[i] = carve<float>(cur, sizes[i]);
     }
     const size_t io_bytes = 256 * 5 + (size_t)(2 * max_streams + max_tokens + 2) * sizeof(int);
