@@ -5,6 +5,8 @@
 // (model.py:89, :346-356, :391), token shift model.py:98-105 (sign of
 // x + (x - x_prev) * mu), the carried `previous` of model.py:197 and the
 // gated output norm of model.py:195-196.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 
@@ -16,21 +18,44 @@ constexpr int kWave = 64;
 // One wave per row; rows of width d <= 64 * kMaxPerLane.
 constexpr int kMaxPerLane = 32;
 
+// A row's loads -- values, affine, gate -- are all issued ahead of the two
+// reductions, so the kernel is one memory round trip (333 rows of 640: 4.2 us,
+// 6.7 with the affine and the gate read behind the reductions).  keep_n rows of
+// keep_src are copied to keep_dst[slot[b]] on the way: save_prev without a launch
+// of its own (4.5 us a layer), once the readers of keep_dst are done.
 template <int PER>
-__global__ void __launch_bounds__(256) layernorm_kernel(const float *x, int M, int d, const float *gamma,
-                                                        const float *beta, const float *gate, float *out) {
+__global__ void __launch_bounds__(256) layernorm_kernel(const float *__restrict__ x, int M, int d,
+                                                        const float *__restrict__ gamma,
+                                                        const float *__restrict__ beta,
+                                                        const float *__restrict__ gate, float *__restrict__ out,
+                                                        const float *__restrict__ keep_src,
+                                                        float *__restrict__ keep_dst, const int *__restrict__ slot,
+                                                        int keep_n) {
+    for (int b = blockIdx.x; b < keep_n; b += gridDim.x) {
+        float *dst = keep_dst + (size_t)(slot ? slot[b] : b) * d;
+        for (int c = threadIdx.x; c < d; c += 256) dst[c] = keep_src[(size_t)b * d + c];
+    }
     const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     if (row >= M) return;
     const float *xr = x + (size_t)row * d;
-    float v[PER];
+    const float *grow = gate ? gate + (size_t)row * d : nullptr;
+    float v[PER], gm[PER], bt[PER], gt[PER];
     float sum = 0.0f;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
         const int c = lane + e * kWave;
         v[e] = c < d ? xr[c] : 0.0f;
-        sum += v[e];
     }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        const int c = lane + e * kWave;
+        gm[e] = c < d ? gamma[c] : 0.0f;
+        bt[e] = c < d ? beta[c] : 0.0f;
+        gt[e] = grow && c < d ? grow[c] : 1.0f;
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) sum += v[e];
     const float mean = wave_sum(sum) / (float)d;
     float sq = 0.0f;
 #pragma unroll
@@ -41,13 +66,12 @@ __global__ void __launch_bounds__(256) layernorm_kernel(const float *x, int M, i
     }
     const float rstd = rsqrtf(wave_sum(sq) / (float)d + 1e-5f);
     float *orow = out + (size_t)row * d;
-    const float *grow = gate ? gate + (size_t)row * d : nullptr;
 #pragma unroll
     for (int e = 0; e < PER; ++e) {
         const int c = lane + e * kWave;
         if (c < d) {
-            float y = (v[e] - mean) * rstd * gamma[c] + beta[c];
-            if (grow) y *= grow[c];
+            float y = (v[e] - mean) * rstd * gm[e] + bt[e];
+            if (grow) y *= gt[e];
             orow[c] = y;
         }
     }
@@ -302,19 +326,22 @@ int grid_for(size_t n, int block) {
 }  // namespace
 
 hipError_t launch_layernorm(const float *x, int M, int d, const float *gamma, const float *beta, const float *gate,
-                            float *out, hipStream_t stream) {
+                            float *out, hipStream_t stream, const float *keep_src, float *keep_dst, const int *slot,
+                            int keep_n) {
     if (M <= 0) return hipSuccess;
     const int per = (d + kWave - 1) / kWave;
     const dim3 grid((M + 3) / 4), block(256);
-    if (per <= 2) hipLaunchKernelGGL(layernorm_kernel<2>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else if (per <= 4) hipLaunchKernelGGL(layernorm_kernel<4>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else if (per <= 8) hipLaunchKernelGGL(layernorm_kernel<8>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else if (per <= 10) hipLaunchKernelGGL(layernorm_kernel<10>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else if (per <= 16) hipLaunchKernelGGL(layernorm_kernel<16>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else if (per <= kMaxPerLane)
-        hipLaunchKernelGGL(layernorm_kernel<kMaxPerLane>, grid, block, 0, stream, x, M, d, gamma, beta, gate, out);
-    else return hipErrorInvalidValue;
-    return hipGetLastError();
+    auto go = [&](auto k) {
+        hipLaunchKernelGGL(k, grid, block, 0, stream, x, M, d, gamma, beta, gate, out, keep_src, keep_dst, slot, keep_n);
+        return hipGetLastError();
+    };
+    if (per <= 2) return go(layernorm_kernel<2>);
+    if (per <= 4) return go(layernorm_kernel<4>);
+    if (per <= 8) return go(layernorm_kernel<8>);
+    if (per <= 10) return go(layernorm_kernel<10>);
+    if (per <= 16) return go(layernorm_kernel<16>);
+    if (per <= kMaxPerLane) return go(layernorm_kernel<kMaxPerLane>);
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_ln_shift(float *x, int n, int d, const float *gamma, const float *beta, float *prev_state,
@@ -361,7 +388,11 @@ hipError_t launch_ln_shift_seq(const float *x, int Bn, int T, int d, const float
                                const float *prev_state, const int *slot, const float *mix6, float *out6,
                                size_t out_stride, float *last_xn, hipStream_t stream) {
     if (Bn <= 0 || T <= 0) return hipSuccess;
-    constexpr int R = 16;  // tokens per wave: one extra LayerNorm per 16 rows
+    // Tokens per wave: a run costs one extra LayerNorm and its rows follow each
+    // other, so short prefills take short runs, down to one token, until they
+    // have a wave per SIMD (333 tokens: 6.4 us, 25.6 in runs of 16 on 6 workgroups);
+    // 16 where there are rows for it (16384: 57 us).  Same bits for any R.
+    const int R = std::max(1, std::min(16, (int)((long long)Bn * T / 1024)));
     const int waves = Bn * ((T + R - 1) / R), per = (d + kWave - 1) / kWave;
     const dim3 grid((waves + 3) / 4), block(256);
     if (per <= 2)

@@ -391,22 +391,25 @@ int gemm(Engine &e, hipStream_t st, int M, int N, int K, const float *A, int lda
 // LayerNorm(A) [* gate] -> Linear.  Short products (M <= 64) fold the norm into
 // the GEMM's A prologue; otherwise -- and for the wide LM head, whose many
 // workgroups would each recompute the row statistics -- the normed rows go
-// through `scratch` first.
+// through `scratch` first (keep_*: launch_layernorm's copy; a save_prev of its
+// own where the norm is fused).
 int ln_gemm(Engine &e, hipStream_t st, int M, int N, int K, const float *A, int lda, const float *gamma,
             const float *beta, const float *gate, float *scratch, const float *W, float *C, int ldc,
             const float *bias = nullptr, const float *residual = nullptr, int ldr = 0, bool silu_pair = false,
-            bool a_tiled = false, bool c_tiled = false) {
+            bool a_tiled = false, bool c_tiled = false, const float *keep_src = nullptr, float *keep_dst = nullptr,
+            const int *keep_slot = nullptr, int keep_n = 0) {
     // Wide N fuses only where the wide decode kernel runs (fp32 W, 32 < M, K <= 640).
     if (M <= 64 && K % 4 == 0 && K <= 1024 && (N <= 8192 || (M > 32 && K <= 640 && !e.w_h))) {
         GemmParams p = make_gemm(e, M, N, K, A, lda, W, K, C, ldc, bias, ACT_NONE, residual, ldr, silu_pair);
         p.ln_gamma = gamma; p.ln_beta = beta; p.a_gate = gate; p.ldg = gate ? lda : 0;
         p.a_tiled = a_tiled; p.c_tiled = c_tiled;
         ENG_TRY(launch_gemm(p, st), "ln gemm");
+        if (keep_n) ENG_TRY(launch_save_prev(keep_src, keep_n, 1, lda, keep_dst, keep_slot, st), "save_prev");
         return YUF_OK;
     }
     if (a_tiled || c_tiled) return fail(YUF_ERR_INVALID, "ln_gemm: tiled operands need the fused path");
     if (lda != K) return fail(YUF_ERR_INVALID, "ln_gemm: strided rows need the fused path");
-    ENG_TRY(launch_layernorm(A, M, K, gamma, beta, gate, scratch, st), "layernorm");
+    ENG_TRY(launch_layernorm(A, M, K, gamma, beta, gate, scratch, st, keep_src, keep_dst, keep_slot, keep_n), "layernorm");
     return gemm(e, st, M, N, K, scratch, K, W, K, C, ldc, bias, ACT_NONE, residual, ldr, silu_pair);
 }
 
@@ -560,6 +563,7 @@ int forward_pass(Engine &e, const Act &a, int n, int Tc, float *logits, int mode
         float *wkv = e.st_wkv + (size_t)l * e.max_streams * e.wkv_floats();
         float *ros = e.st_rosa + (size_t)l * e.max_streams * D;
         // TimeMix
+        int keep_n = 0;  // rows of a.hl that still go to prev
         if (Tc == 1 && d <= 1024) {
             // The previous layer's FFN output may be pending as K-split partials.
             const int np = ffn_split && l > 0 ? kFfnParts : 0;
@@ -567,10 +571,11 @@ int forward_pass(Engine &e, const Act &a, int n, int Tc, float *logits, int mode
                                     np ? a.kpart : nullptr, a.kplane, np, tl, st), "ln_shift");
         } else if (d <= 1024) {
             // LayerNorm + token shift in one pass; the last normed row of each
-            // stream goes through a.hl (free until the LM head) to prev.
+            // stream goes through a.hl (free until the LM head) to prev, copied
+            // by the output norm's launch below.
             ENG_TRY(launch_ln_shift_seq(a.h, n, Tc, d, w.ln_t_w, w.ln_t_b, prev, a.slots, w.mix6, a.mix, plane, a.hl,
                                         st), "ln_shift_seq");
-            ENG_TRY(launch_save_prev(a.hl, n, 1, d, prev, a.slots, st), "save_prev");
+            keep_n = n;
         } else {
             ENG_TRY(launch_layernorm(a.h, M, d, w.ln_t_w, w.ln_t_b, nullptr, a.xn, st), "ln_time");
             ENG_TRY(launch_token_shift(a.xn, n, Tc, d, prev, a.slots, w.mix6, a.mix, plane, st), "token_shift");
@@ -623,7 +628,7 @@ int forward_pass(Engine &e, const Act &a, int n, int Tc, float *logits, int mode
             e.wkv_probe_set = true;
         }
         if ((rc = ln_gemm(e, st, M, d, d, a.y, d, w.ln_o_w, w.ln_o_b, a.g, a.z, w.w_o, a.h, d, nullptr, a.h, d, false,
-                          tl)) != YUF_OK)
+                          tl, false, a.hl, prev, a.slots, keep_n)) != YUF_OK)
             return rc;
         // ROSA
         if ((rc = ln_gemm(e, st, M, 3 * D, d, a.h, d, w.ln_r_w, w.ln_r_b, nullptr, a.xn, w.rosa_w3, a.rosa3, 3 * D,

@@ -228,8 +228,10 @@ hipError_t launch_embed(const int *tokens, int M, const float *table, int d, int
                         int *bad_token_flag, hipStream_t stream);
 // out = LayerNorm(x) * gamma + beta, rows of width d (eps 1e-5); optional
 // row gather (`rows`), optional multiply by `gate` after the affine.
+// keep_n > 0: keep_dst[slot[b]] = keep_src[b] for b < keep_n as well (rows of width d).
 hipError_t launch_layernorm(const float *x, int M, int d, const float *gamma, const float *beta,
-                            const float *gate, float *out, hipStream_t stream);
+                            const float *gate, float *out, hipStream_t stream, const float *keep_src = nullptr,
+                            float *keep_dst = nullptr, const int *slot = nullptr, int keep_n = 0);
 // Token shift: six outputs out[c][m, :] = x[m] + (x[m] - x_prev(m)) * mix[c],
 // x_prev(m) = x[m - 1] inside a row of T tokens, prev_state[slot[b]] at t = 0.
 hipError_t launch_token_shift(const float *x, int Bn, int T, int d, const float *prev_state,
