@@ -441,6 +441,26 @@ hipError_t launch_rosa_gates(float *x, int M, int D, int ld, hipStream_t stream)
     return hipGetLastError();
 }
 
+// A run of rows of each of several equally spaced planes of up to three arrays
+// to zero: one launch for a whole recurrent state (42 fills of ~1.8 us each and
+// their gaps for 14 layers before).
+__global__ void clear_rows_kernel(ClearRows a) {
+    for (int q = 0; q < 3; ++q) {
+        const size_t n = a.count[q] * (size_t)a.planes;
+        for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+            const size_t l = i / a.count[q];
+            a.base[q][l * a.stride[q] + (i - l * a.count[q])] = 0.0f;
+        }
+    }
+}
+
+hipError_t launch_clear_rows(const ClearRows &a, hipStream_t stream) {
+    const size_t n = std::max({a.count[0], a.count[1], a.count[2]}) * (size_t)a.planes;
+    if (n == 0) return hipSuccess;
+    hipLaunchKernelGGL(clear_rows_kernel, dim3(std::min(grid_for(n, 256), 4096)), dim3(256), 0, stream, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill(float *p, size_t n, float value, hipStream_t stream) {
     if (n == 0) return hipSuccess;
     hipLaunchKernelGGL(fill_kernel, dim3(grid_for(n, 256)), dim3(256), 0, stream, p, n, value);

@@ -1403,14 +1403,16 @@ extern "C" int yuf_state_reset(yuf_engine *eng, int slot) {
     Engine &e = eng->e;
     if (slot < -1 || slot >= e.max_streams) return fail(YUF_ERR_RANGE, "slot out of range");
     const int first = slot < 0 ? 0 : slot, count = slot < 0 ? e.max_streams : 1;
-    for (int l = 0; l < e.s.layers; ++l) {
-        struct { float *base; size_t per; } parts[3] = {
-            {e.st_prev + (size_t)l * e.max_streams * e.s.d, (size_t)e.s.d},
-            {e.st_wkv + (size_t)l * e.max_streams * e.wkv_floats(), e.wkv_floats()},
-            {e.st_rosa + (size_t)l * e.max_streams * e.s.rosa, (size_t)e.s.rosa}};
-        for (auto &p : parts)
-            ENG_TRY(launch_fill(p.base + (size_t)first * p.per, (size_t)count * p.per, 0.0f, e.stream), "state reset");
+    ClearRows rows;
+    rows.planes = e.s.layers;
+    struct { float *base; size_t per; } parts[3] = {
+        {e.st_prev, (size_t)e.s.d}, {e.st_wkv, e.wkv_floats()}, {e.st_rosa, (size_t)e.s.rosa}};
+    for (int q = 0; q < 3; ++q) {
+        rows.base[q] = parts[q].base + (size_t)first * parts[q].per;
+        rows.stride[q] = (size_t)e.max_streams * parts[q].per;
+        rows.count[q] = (size_t)count * parts[q].per;
     }
+    ENG_TRY(launch_clear_rows(rows, e.stream), "state reset");
     ENG_TRY(hipStreamSynchronize(e.stream), "state reset sync");
     return YUF_OK;
 }

@@ -260,6 +260,13 @@ hipError_t launch_save_prev(const float *x, int Bn, int T, int d, float *prev_st
 hipError_t launch_gather_last(const float *x, int Bn, int T, int d, float *out, hipStream_t stream);
 // state blob pack/unpack and clearing.
 hipError_t launch_fill(float *p, size_t n, float value, hipStream_t stream);
+// base[q][l * stride[q] + i] = 0 for l < planes, i < count[q].
+struct ClearRows {
+    float *base[3] = {};
+    size_t stride[3] = {}, count[3] = {};
+    int planes = 0;
+};
+hipError_t launch_clear_rows(const ClearRows &a, hipStream_t stream);
 // In place on rows [cand | write | read_raw] of stride ld: cand <- e, write <- gate.
 hipError_t launch_rosa_gates(float *x, int M, int D, int ld, hipStream_t stream);
 
