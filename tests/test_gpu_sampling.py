@@ -210,6 +210,32 @@ def test_full_vocab_edge_rows(vocab):
                                           err_msg=f"top_k={top_k} top_p={top_p} step {step}")
 
 
+@pytest.mark.parametrize("vocab", [1, 2, 255, 256, 1023, 1024, 1025, 16385])
+def test_full_vocab_sort_edges(vocab):
+    """The radix sort at the edges of its rounds, on rows whose 8-bit key digits
+    are all alike in some passes and dense in others (values one float step
+    apart, two exponents, every value once in falling order, ties): the host's
+    tokens."""
+    rng = np.random.default_rng(700 + vocab)
+    steps = np.arange(vocab, dtype=np.uint32)
+    x = np.stack([
+        (np.uint32(0x3F800000) + rng.permutation(steps)).view(np.float32),
+        np.where(rng.random(vocab) < 0.5, 1.0, -2.0).astype(np.float32),
+        np.linspace(3.0, -3.0, vocab, dtype=np.float32),
+        (rng.standard_normal(vocab) * 2.0).astype(np.float32),
+    ])
+    logits = torch.from_numpy(x).cuda()
+    tokens = torch.empty(4, dtype=torch.int32, device="cuda")
+    host = [Mt19937(40 + s) for s in range(4)]
+    dev = [g.copy() for g in host]
+    for step in range(2):
+        q, _ = _exact_draws(dev, vocab, vocab)
+        sample_device_masked(logits, tokens, 1.0, 0.9, 0, exp_draws=q)
+        torch.cuda.synchronize()
+        expect = [sample_token(x[s], 1.0, 0.9, host[s], top_k=0) for s in range(4)]
+        np.testing.assert_array_equal(tokens.cpu().numpy(), np.array(expect), err_msg=f"step {step}")
+
+
 def test_full_vocab_counter_mode_stays_in_the_nucleus():
     """Counter draws (no host work): every token lies in the host's nucleus of
     the masked row, and a near-flat row spreads over many ids."""

@@ -432,10 +432,13 @@ __global__ void __launch_bounds__(NTH) sample_kernel(SampleParams p) {
 // 16-lane order, so every value's position matters.  One workgroup of 1024
 // threads per stream:
 //   1. mask + scale, then a stable LSD radix sort of (key, token id) in LDS:
-//      4-bit digits, eight passes (a pass whose digit is the same for every
-//      value is skipped); element e of a pass is handled by thread e % 1024
-//      in round e / 1024, so a ballot ranks it among its wave's equal digits
-//      and an exclusive scan over (digit, round, wave) counts places it;
+//      8-bit digits, four passes (a pass whose digit is the same for every
+//      value is skipped).  The sort is bound by vector instructions of the one
+//      CU, about in proportion to digit passes: a wave owns R x 64 consecutive
+//      positions, eight ballots rank a round's lanes among their equal digits,
+//      a running count per (digit, wave) in LDS carries the rank over the
+//      rounds, and what it ends at, scanned in (digit, wave) order, places the
+//      elements;
 //   2. e_i = exp(x_i - max) rounded once to float, their sum by 16 lanes in
 //      the host's order, p_i = e_i * (1 / sum);
 //   3. the cut (float)cum_i - p_i > top_p with cum the host's sequential
@@ -453,6 +456,7 @@ constexpr int kFullThreads = 1024;
 constexpr int kFullWaves = kFullThreads / 64;
 constexpr int kFullMaxV = 24576;
 constexpr int kFullMaxRounds = kFullMaxV / kFullThreads;
+constexpr int kFullDigits = 256;  // of a sort pass
 constexpr uint16_t kDropBit = 0x8000;  // top-p cut flag in the id array (ids < 32768)
 
 // Ascending keys = the host's descending order of values; -0.0 counts as +0.0
@@ -496,16 +500,32 @@ __device__ __forceinline__ T block_excl_scan(T x, T *sh, int lane, int wave) {
 __device__ __forceinline__ float sum16_lds(const float *e, const uint16_t *ids, int n, bool cut, int lane) {
     float acc = 0.0f;
     if (lane < 16) {
-        int i = lane;
-        for (; i + 7 * 16 < n; i += 8 * 16) {
-            float v[8];
+        // The chain of additions is what is left: the next batch's reads are in
+        // flight while a batch is added.
+        constexpr int kU = 16;
+        auto load = [&](float (&v)[kU], int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                v[u] = e[i + 16 * u];
-                if (cut && (ids[i + 16 * u] & kDropBit)) v[u] = 0.0f;
+            for (int u = 0; u < kU; ++u) v[u] = e[i + 16 * u];
+            if (cut) {
+#pragma unroll
+                for (int u = 0; u < kU; ++u)
+                    if (ids[i + 16 * u] & kDropBit) v[u] = 0.0f;
             }
+        };
+        auto add = [&](const float (&v)[kU]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u) acc += v[u];
+            for (int u = 0; u < kU; ++u) acc += v[u];
+        };
+        int i = lane;
+        const int batches = n / (16 * kU);  // whole ones of every lane
+        float v0[kU], v1[kU];
+        if (batches > 0) load(v0, i);
+        for (int b = 0; b < batches; b += 2) {
+            if (b + 1 < batches) load(v1, i + 16 * kU);
+            add(v0);
+            if (b + 2 < batches) load(v0, i + 32 * kU);
+            if (b + 1 < batches) add(v1);
+            i += 16 * kU * min(2, batches - b);
         }
         for (; i < n; i += 16) acc += (cut && (ids[i] & kDropBit)) ? 0.0f : e[i];
     }
@@ -520,15 +540,16 @@ __device__ __forceinline__ float sum16_lds(const float *e, const uint16_t *ids, 
 __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(SampleParams p) {
     __shared__ uint32_t skey[kFullMaxV];  // sort keys; after the sort, e_i as float bits
     __shared__ uint16_t sidx[kFullMaxV];  // token ids; kDropBit once cut by top-p
-    // Digit counts, then their offsets, per (digit, round, wave); before the
-    // sort, the blocked-id bitmap of the generation mask.
-    __shared__ uint32_t scnt32[16 * kFullMaxRounds * kFullWaves / 2];
+    // Digit counts, then their offsets, per (digit, wave); before the sort, the
+    // blocked-id bitmap of the generation mask.
+    __shared__ uint32_t scnt32[kFullDigits * kFullWaves / 2];
     __shared__ uint64_t sh_u64[kFullWaves];
     __shared__ double sh_f64[kFullWaves];
     __shared__ int sh_int[kFullWaves], sh_int2[kFullWaves];
     __shared__ float sh_flt[kFullWaves];
     __shared__ float sh_sum;
-    static_assert(kSampleMaskWords <= 16 * kFullMaxRounds * kFullWaves / 2, "bitmap fits the count array");
+    static_assert(kSampleMaskWords <= kFullDigits * kFullWaves / 2, "bitmap fits the count array");
+    static_assert(kFullDigits * kFullWaves == 4 * kFullThreads, "four counts a thread");
     uint16_t *scnt = reinterpret_cast<uint16_t *>(scnt32);
     float *se = reinterpret_cast<float *>(skey);
 
@@ -571,73 +592,71 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(SampleParams 
     }
     __syncthreads();
 
-    // Stable LSD radix sort of (key, id), 4 bits per pass.
-    const int n_cnt = 16 * R * kFullWaves;
-    const int per = (n_cnt + kFullThreads - 1) / kFullThreads;
-    for (int shift = 0; shift < 32; shift += 4) {
+    // Stable LSD radix sort of (key, id), 8 bits per pass.
+    const int e0 = wave * R * 64 + lane;  // this lane's position in round 0 of its wave's run
+    for (int shift = 0; shift < 32; shift += 8) {
+        const uint32_t d0 = (skey[0] >> shift) & 255u;
         uint32_t kr[kFullMaxRounds], ir[kFullMaxRounds];
+        bool one_digit = true;
 #pragma unroll
         for (int r = 0; r < kFullMaxRounds; ++r)
             if (r < R) {
-                kr[r] = skey[r * kFullThreads + tid];
-                ir[r] = sidx[r * kFullThreads + tid];
+                kr[r] = skey[e0 + r * 64];
+                ir[r] = sidx[e0 + r * 64];
+                one_digit &= ((kr[r] >> shift) & 255u) == d0;
             }
+        // A digit that every element shares leaves the order unchanged.
+        if (lane == 0) sh_int2[wave] = 1;
+        if (!one_digit) sh_int2[wave] = 0;
+        reinterpret_cast<uint2 *>(scnt32)[tid] = make_uint2(0u, 0u);
+        __syncthreads();
+        int same_digit = 1;
+#pragma unroll
+        for (int w = 0; w < kFullWaves; ++w) same_digit &= sh_int2[w];
+        if (same_digit) {
+            __syncthreads();
+            continue;
+        }
 #pragma unroll
         for (int r = 0; r < kFullMaxRounds; ++r)
             if (r < R) {
-                const uint32_t dg = (kr[r] >> shift) & 15u;
-                uint64_t bal[4];
+                const uint32_t dg = (kr[r] >> shift) & 255u;
                 uint64_t same = ~0ull;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    bal[b] = __ballot((dg >> b) & 1u);
-                    same &= ((dg >> b) & 1u) ? bal[b] : ~bal[b];
+                for (int b = 0; b < 8; ++b) {
+                    const uint64_t bal = __ballot((dg >> b) & 1u);
+                    const uint64_t bit = (uint64_t)(int64_t)((int32_t)(dg << (31 - b)) >> 31);
+                    same &= ~(bal ^ bit);
                 }
-                ir[r] |= (uint32_t)__popcll(same & lt_mask) << 16;
-                if (lane < 16) {
-                    uint64_t m = ~0ull;
-#pragma unroll
-                    for (int b = 0; b < 4; ++b) m &= ((lane >> b) & 1) ? bal[b] : ~bal[b];
-                    scnt[(lane * R + r) * kFullWaves + wave] = (uint16_t)__popcll(m);
-                }
+                // Rank among the wave's equal digits so far; the last of a round's equal lanes moves the count on.
+                const uint32_t rank = scnt[dg * kFullWaves + wave] + (uint32_t)__popcll(same & lt_mask);
+                // (A wave's LDS accesses complete in order: the barriers only keep the compiler's.)
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+                __builtin_amdgcn_wave_barrier();
+                if ((same >> lane) == 1ull) scnt[dg * kFullWaves + wave] = (uint16_t)(rank + 1u);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+                __builtin_amdgcn_wave_barrier();
+                ir[r] |= rank << 16;
             }
         __syncthreads();
-        // Exclusive scan of the counts in (digit, round, wave) order.
+        // Exclusive scan of the counts in (digit, wave) order, four a thread
+        // (all but the total fit 16 bits: at most kFullMaxV elements).
         {
-            int loc[8];
-            int tot = 0;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int c = tid * per + j;
-                loc[j] = (j < per && c < n_cnt) ? (int)scnt[c] : 0;
-                tot += loc[j];
-            }
-            int base = block_excl_scan(tot, sh_int, lane, wave);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int c = tid * per + j;
-                if (j < per && c < n_cnt) scnt[c] = (uint16_t)base;
-                base += loc[j];
-            }
+            const uint2 c = reinterpret_cast<const uint2 *>(scnt32)[tid];
+            const uint32_t c0 = c.x & 0xffffu, c1 = c.x >> 16, c2 = c.y & 0xffffu, c3 = c.y >> 16;
+            const uint32_t base = (uint32_t)block_excl_scan((int)(c0 + c1 + c2 + c3), sh_int, lane, wave);
+            const uint32_t o1 = base + c0, o2 = o1 + c1, o3 = o2 + c2;
+            reinterpret_cast<uint2 *>(scnt32)[tid] = make_uint2(base | (o1 << 16), o2 | (o3 << 16));
         }
         __syncthreads();
-        // A digit that every element shares leaves the order unchanged.
-        bool trivial = false;
-        const int np = R * kFullThreads;
-        for (int d = 0; d < 16; ++d) {
-            const int lo = scnt[d * R * kFullWaves], hi = d < 15 ? (int)scnt[(d + 1) * R * kFullWaves] : np;
-            trivial |= hi - lo == np;
-        }
-        if (!trivial) {
 #pragma unroll
-            for (int r = 0; r < kFullMaxRounds; ++r)
-                if (r < R) {
-                    const uint32_t dg = (kr[r] >> shift) & 15u;
-                    const int pos = (int)scnt[(dg * R + r) * kFullWaves + wave] + (int)(ir[r] >> 16);
-                    skey[pos] = kr[r];
-                    sidx[pos] = (uint16_t)(ir[r] & 0xffffu);
-                }
-        }
+        for (int r = 0; r < kFullMaxRounds; ++r)
+            if (r < R) {
+                const uint32_t dg = (kr[r] >> shift) & 255u;
+                const int pos = (int)scnt[dg * kFullWaves + wave] + (int)(ir[r] >> 16);
+                skey[pos] = kr[r];
+                sidx[pos] = (uint16_t)(ir[r] & 0xffffu);
+            }
         __syncthreads();
     }
 
