@@ -65,6 +65,27 @@ def test_wkv7_many_heads_one_workgroup_each(size, wkv_kernel):
     np.testing.assert_allclose(s.cpu().numpy(), se.numpy(), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("split", ["1", "2", "4"])
+@pytest.mark.parametrize("size", [32, 40, 48, 64])
+@pytest.mark.parametrize("steps", [1, 15, 33, 80])
+def test_wkv7_split_heads(size, steps, split, monkeypatch):
+    """A head over two workgroups or one per 16 value rows, of two to
+    four tiles with a half or whole last one: the oracle's outputs and states, for the
+    fewest chunks a pipeline of five can meet (one, ragged) and for several."""
+    from yufmusicgen_amd.ops import rwkv7_scan
+
+    print(f"wkv7 split={split} N={size} T={steps}", flush=True)
+    monkeypatch.setenv("YUF_WKV7_KERNEL", "chunked")
+    monkeypatch.setenv("YUF_WKV7_SPLIT", split)
+    arrs = wkv_inputs(500 + size + steps, 2, steps, 5, size)
+    s0 = np.random.default_rng(size + 7).standard_normal((2, 5, size, size)).astype(np.float32) * 0.3
+    y, s = rwkv7_scan(*(_dev(x) for x in arrs), state=_dev(s0))
+    ye, se = _oracle_wkv(arrs, s0)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(y.cpu().numpy(), ye.numpy(), rtol=RTOL, atol=ATOL)
+    np.testing.assert_allclose(s.cpu().numpy(), se.numpy(), rtol=RTOL, atol=ATOL)
+
+
 def test_wkv7_reference_golden(golden_dir):
     from yufmusicgen_amd.ops import rwkv7_scan
 

@@ -83,18 +83,26 @@ __device__ __forceinline__ void buf_store4(floatx4 v, __amdgpu_buffer_rsrc_t rsr
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rsrc, byte_offset, 0, 0);
 }
 
-template <int NB, bool SPLIT>
+// VT: value tiles of one workgroup of a split head, 0 for whole heads.
+template <int NB, int VT>
 struct Lds {
-    // Ring depths: a split workgroup's Y wave reads chunk c - 1's ring entries
-    // while stage A writes chunk c + 3 and stage B1 chunk c + 2.
-    static constexpr int kRA = SPLIT ? 5 : 4, kRG = SPLIT ? 4 : 3;
+    // Ring depths: a split workgroup's Y wave reads chunk c - 1's R~, V, Qb and
+    // Qk while stage A writes chunk c + 3 and stage B1 chunk c + 2.  kTight: R~
+    // and V^T in a ring of their own, five deep beside ring A's four, and V^T rows
+    // of the workgroup's tiles only, for the LDS of NB = 4; elsewhere part of ring
+    // A's slots (8 x 2048 x 16 x 40: 153 us, 159 with the rings apart).
+    static constexpr bool kTight = NB == 4 && VT > 0;
+    static constexpr int kRA = VT && !kTight ? 5 : 4, kRV = VT ? 5 : 4, kRG = VT ? 4 : 3;
     static constexpr int NP = 16 * NB;        // padded head size
     static constexpr int SA = NP + 4;         // row stride of [token][column] tiles
-    // Ring A (4 chunks in flight): A~, R~ [16][SA]; B^^T, K^^T [NP][kST]; g_15 [NP];
-    // V^T [NP][kST] (value row, token).
-    static constexpr int oAs = 0, oRs = 16 * SA, oBhT = 32 * SA, oKhT = oBhT + NP * kST, oGl = oKhT + NP * kST;
-    static constexpr int oV = oGl + NP;
-    static constexpr int kSlotA = oV + NP * kST;
+    // Ring A (kRA): A~ [16][SA]; R~ unless kTight; B^^T, K^^T [NP][kST]; g_15 [NP];
+    // V^T [NP][kST] (value row, token) unless kTight.
+    static constexpr int oAs = 0, oBhT = (kTight ? 16 : 32) * SA, oKhT = oBhT + NP * kST, oGl = oKhT + NP * kST;
+    static constexpr int oRs = kTight ? 0 : 16 * SA, oV = kTight ? 16 * SA : oGl + NP;
+    static constexpr int kStrideA = kTight ? oGl + NP : oV + NP * kST;
+    // Ring V (kTight, kRV): R~ [16][SA]; V^T [value rows of the workgroup][kST].
+    static constexpr int kStrideV = kTight ? oV + 16 * VT * kST : kStrideA;
+    static constexpr int kRings = kRA * kStrideA + (kTight ? kRV * kStrideV : 0);
     // Ring G (3): Gab^T [s][t], P, Qb, Qk [t][s], all [16][kST].
     static constexpr int oGabT = 0, oP = 16 * kST, oQb = 32 * kST, oQk = 48 * kST, kSlotG = 64 * kST;
     // Ring T (2): (I - Gab)^{-1} [16][kST].
@@ -106,9 +114,11 @@ struct Lds {
     static constexpr int kSlotR = 5 * 16 * kST;
     // Split: consumer -> Y wave exchange, [chunk parity][value tile][vector k]
     // [lane] floatx4: k < NB the chunk-start state S0^T rows, k = NB the U tile.
-    static constexpr int kSlotX = SPLIT ? 2 * 2 * 4 * 64 * 4 : 0;
-    static constexpr int kFloats =
-        kRA * kSlotA + kRG * kSlotG + 2 * kSlotT + 2 * kSlotN + NB * kSlotR + kSlotX;
+    static constexpr int kTileX = (NB + 1) * 64;  // floatx4 of one tile
+    static constexpr int kSlotX = 2 * VT * kTileX * 4;
+    static constexpr int kFloats = kRings + kRG * kSlotG + 2 * kSlotT + 2 * kSlotN +
+                                   NB * kSlotR + kSlotX;
+    static_assert(kFloats * 4 <= 160 * 1024, "LDS of one CU");
 };
 
 // Wave roles.  Waves w and w + 4 of a workgroup share a SIMD, and a wave
@@ -127,61 +137,65 @@ template <int NB> struct Roles {
         return r[w];
     }
 };
-// Split heads (two workgroups per head, each with the consumers of its own
-// value tiles and the whole key-space pipeline, NB <= 3).  On gfx950 an fp32
-// MFMA stream and the VALU / LDS work of any wave on the same SIMD run one
+// Split heads (a workgroup per VT value tiles of a head, each with the
+// consumers of its own tiles and the whole key-space pipeline).  On gfx950 an
+// fp32 MFMA stream and the VALU / LDS work of any wave on the same SIMD run one
 // after the other (measured: no overlap), so the work is spread for equal
 // per-SIMD sums: the consumers keep only the state chain (X, U, the state
 // update) and hand the chunk-start state and U to a Y wave that forms the
-// outputs one chunk later.  NB = 3: cons0 + A0, cons1 + A1, B1 + B2, Y + A2.
+// outputs one chunk later.  NB = 3, VT = 2: cons0 + A0, cons1 + A1, B1 + B2,
+// Y + A2; NB = 4, VT = 1: cons0 + A1, B1 + Y, B2 + A2, A0 + A3; NB = 4, VT = 2:
+// three stage-A waves on one SIMD, cons0 + A1, cons1 + B2, B1 + Y.
 // Consumer roles past the workgroup's tile count idle (they keep the barrier
 // count only).
-template <int NB> struct SplitRoles {
-    static constexpr int kWaves = NB == 2 ? 6 : 8;
+template <int NB, int VT> struct RoleMap {
+    static_assert(VT == 0 || (NB == 2 && VT == 1) || (NB == 3 && VT <= 2) || (NB == 4 && VT <= 2), "wave roles");
+    static constexpr int kWaves = VT == 0 ? Roles<NB>::kWaves : NB == 2 ? 6 : NB == 3 ? 6 + VT : 7 + VT;
     __device__ static int of(int w) {
         constexpr int A = kRoleA;
+        if constexpr (VT == 0) return Roles<NB>::of(w);
         if constexpr (NB == 2) { constexpr int r[] = {0, kRoleB1, kRoleY, A, A + 1, kRoleB2}; return r[w]; }
-        constexpr int r[] = {0, 1, kRoleB1, kRoleY, A, A + 1, kRoleB2, A + 2};
+        if constexpr (NB == 3 && VT == 1) { constexpr int r[] = {0, kRoleB1, kRoleB2, A, A + 1, kRoleY, A + 2}; return r[w]; }
+        if constexpr (NB == 3) { constexpr int r[] = {0, 1, kRoleB1, kRoleY, A, A + 1, kRoleB2, A + 2}; return r[w]; }
+        if constexpr (VT == 1) { constexpr int r[] = {0, kRoleB1, kRoleB2, A, A + 1, kRoleY, A + 2, A + 3}; return r[w]; }
+        constexpr int r[] = {A, 0, 1, kRoleB1, A + 1, A + 2, kRoleB2, kRoleY, A + 3};
         return r[w];
     }
 };
-template <int NB, bool SPLIT> struct RoleMap : Roles<NB> {};
-template <int NB> struct RoleMap<NB, true> : SplitRoles<NB> {
-    static_assert(NB == 2 || NB == 3, "split heads need NB in {2, 3}");
-};
 
-// SPLIT: two workgroups per head; the first owns value tiles [0, (NB + 1) / 2),
-// the second the rest.
+// VT > 0: workgroup `part` of a head owns value tiles [VT part, VT part + VT).
 // HALF (N % 16 == 8): the last key tile holds 8 keys.  Its accumulator row
 // m = 4 g + r stands for key 16 (NB - 1) + 8 (r >> 1) + 2 g + (r & 1), so the
 // real keys sit in registers r = 0, 1 of every lane group, and every product
 // over the keys takes k-steps r = 0, 1 only on that tile (k-step r of lane
 // group g: key 2 g + r of the tile) instead of four k-steps of which half
 // would multiply zeros.
-template <int NB, bool PREP, bool SPLIT, bool HALF>
-__global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
+template <int NB, bool PREP, bool SPLIT, bool HALF, int VT>
+__global__ void __launch_bounds__((RoleMap<NB, VT>::kWaves) * kWave)
     wkv7_chunk_kernel(WkvParams p, int N, int units, int per_xcd) {
-    using Ly = Lds<NB, SPLIT>;
-    constexpr int NP = Ly::NP, SA = Ly::SA, kRA = Ly::kRA, kRG = Ly::kRG;
+    using Ly = Lds<NB, VT>;
+    static_assert(SPLIT == (VT > 0), "VT value tiles of a split head");
+    constexpr int NP = Ly::NP, SA = Ly::SA, kRA = Ly::kRA, kRV = Ly::kRV, kRG = Ly::kRG;
     constexpr int kExtra = SPLIT ? 1 : 0;  // iterations after the consumers' last chunk (the Y wave's)
     __shared__ __attribute__((aligned(16))) float lds[Ly::kFloats];
     float *ringA = lds;
-    float *ringG = ringA + kRA * Ly::kSlotA;
+    float *ringV = Ly::kTight ? ringA + kRA * Ly::kStrideA : ringA;
+    float *ringG = ringA + Ly::kRings;
     float *ringT = ringG + kRG * Ly::kSlotG;
     float *ringN = ringT + 2 * Ly::kSlotT;
     float *stageR = ringN + 2 * Ly::kSlotN;
     floatx4 *xch = reinterpret_cast<floatx4 *>(stageR + NB * Ly::kSlotR);  // split only
 
-    // XCD-aware unit index: consecutive units (the two halves of a head, then
+    // XCD-aware unit index: consecutive units (the parts of a head, then
     // consecutive heads of a batch row) share an XCD's L2.
     const int unit = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
     if (unit >= units) return;  // uniform over the workgroup
-    const int flat = SPLIT ? unit >> 1 : unit, part = SPLIT ? unit & 1 : 0;
-    constexpr int kNv0 = SPLIT ? (NB + 1) / 2 : NB;  // value tiles of the first workgroup
-    const int vb0 = part ? kNv0 : 0, nv = part ? NB - kNv0 : kNv0;
+    constexpr int kVt = SPLIT ? VT : NB, kParts = (NB + kVt - 1) / kVt;
+    const int flat = unit / kParts, vb0 = (unit - flat * kParts) * kVt, nv = min(kVt, NB - vb0);
     const int bb = flat / p.H, h = flat - bb * p.H;
+    const int vr0 = Ly::kTight ? 0 : 16 * vb0;  // V^T row of the workgroup's first value row
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    int role = RoleMap<NB, SPLIT>::of(wave);
+    int role = RoleMap<NB, VT>::of(wave);
     if (role < NB && role >= nv) role = kRoleIdle;
     const int g = lane >> 4, li = lane & 15;
     const int T = p.T, HN = p.H * N;
@@ -227,18 +241,18 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
         for (int it = -4; it < n_chunks + kExtra; ++it) {
             const int c = it - 1;
             if (c >= 0) {
-                const float *sA = ringA + (c % kRA) * Ly::kSlotA;
+                const float *sV = ringV + (c % kRV) * Ly::kStrideV;
                 const float *sG = ringG + (c % kRG) * Ly::kSlotG;
-                const floatx4 *xc = xch + (c & 1) * 2 * 4 * 64;
+                const floatx4 *xc = xch + (c & 1) * VT * Ly::kTileX;
                 for (int tl = 0; tl < nv; ++tl) {
                     const int i = 16 * (vb0 + tl) + li;
-                    const floatx4 *xt = xc + tl * 4 * 64;
-                    const floatx4 v = ld4(sA + Ly::oV + i * kST + 4 * g);
+                    const floatx4 *xt = xc + tl * Ly::kTileX;
+                    const floatx4 v = ld4(sV + Ly::oV + (vr0 + 16 * tl + li) * kST + 4 * g);
                     const floatx4 U = xt[NB * 64 + lane];
                     floatx4 Y0 = {0.f, 0.f, 0.f, 0.f}, Y1 = Y0;
 #pragma unroll
                     for (int jb = 0; jb < NB; ++jb) {
-                        const floatx4 r4 = ldk(sA + Ly::oRs + li * SA, jb);
+                        const floatx4 r4 = ldk(sV + Ly::oRs + li * SA, jb);
                         const floatx4 s0 = xt[jb * 64 + lane];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
@@ -290,11 +304,12 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
                 // The state chain only: X = A~ S0^T + P V, U = (I - Gab)^{-1} X,
                 // S^T <- diag(g_15) (S^T + B^^T U + K^^T V); S0^T and U go to the Y wave.
                 const int c = it;
-                const float *sA = ringA + (c % kRA) * Ly::kSlotA;
+                const float *sA = ringA + (c % kRA) * Ly::kStrideA;
                 const float *sG = ringG + (c % kRG) * Ly::kSlotG;
                 const float *sT = ringT + (c & 1) * Ly::kSlotT;
-                floatx4 *xt = xch + ((c & 1) * 2 + role) * 4 * 64;
-                const floatx4 v = ld4(sA + Ly::oV + i * kST + 4 * g);  // V[4 g + r][i]
+                const float *sV = ringV + (c % kRV) * Ly::kStrideV;
+                floatx4 *xt = xch + ((c & 1) * VT + role) * Ly::kTileX;
+                const floatx4 v = ld4(sV + Ly::oV + (vr0 + 16 * role + li) * kST + 4 * g);  // V[4 g + r][i]
                 floatx4 X0 = {0.f, 0.f, 0.f, 0.f}, X1 = X0;
 #pragma unroll
                 for (int jb = 0; jb < NB; ++jb) {
@@ -334,15 +349,16 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
                 }
             } else if (!SPLIT && it >= 0) {
                 const int c = it;
-                const float *sA = ringA + (c % kRA) * Ly::kSlotA;
+                const float *sA = ringA + (c % kRA) * Ly::kStrideA;
                 const float *sG = ringG + (c % kRG) * Ly::kSlotG;
                 const float *sT = ringT + (c & 1) * Ly::kSlotT;
-                const floatx4 v = ld4(sA + Ly::oV + i * kST + 4 * g);  // V[4 g + r][i]
+                const float *sV = ringV + (c % kRV) * Ly::kStrideV;
+                const floatx4 v = ld4(sV + Ly::oV + (vr0 + 16 * role + li) * kST + 4 * g);  // V[4 g + r][i]
                 floatx4 X = {0.f, 0.f, 0.f, 0.f}, Y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int jb = 0; jb < NB; ++jb) {
                     const floatx4 a4 = ldk(sA + Ly::oAs + li * SA, jb);
-                    const floatx4 r4 = ldk(sA + Ly::oRs + li * SA, jb);
+                    const floatx4 r4 = ldk(sV + Ly::oRs + li * SA, jb);
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         if (r >= ksteps(jb)) break;
@@ -418,6 +434,10 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
         __amdgpu_buffer_rsrc_t rs[kIn];
 #pragma unroll
         for (int x = 0; x < kIn; ++x) rs[x] = make_rsrc(src[x] + tok_base, tok_bytes);
+        // This wave's 16 columns of v are value tile `vt` of the head (kTight: kept
+        // where the workgroup owns it).
+        const int vt = role - kRoleA - (Ly::kTight ? vb0 : 0);
+        const bool own_v = !Ly::kTight || (vt >= 0 && vt < nv);
         float kk_w = 0.0f, ka_w = 0.0f;
         if constexpr (PREP) {
             const bool col_ok = j < N;
@@ -455,10 +475,12 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
         // Chunk c (iteration c - 3); its set is reloaded with chunk c + 2.
         auto body = [&](int c, floatx4 (&ld)[kIn], bool load_next) {
             {
-                float *sA = ringA + (c % kRA) * Ly::kSlotA;
+                float *sA = ringA + (c % kRA) * Ly::kStrideA, *sV = ringV + (c % kRV) * Ly::kStrideV;
                 transpose(ld);
+                if (own_v) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) sA[Ly::oV + (lc0 + e) * kST + li] = ld[kT][e];
+                    for (int e = 0; e < 4; ++e) sV[Ly::oV + (16 * vt + 4 * qg + e) * kST + li] = ld[kT][e];
+                }
                 if (load_next) load_chunk(ld, c + 2);
                 const int nt = min(kC, T - c * kC);
                 float av[4], bv[4], kv[4], rv[4], dv[4];
@@ -509,7 +531,7 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
                 const float R = __uint_as_float(sw32[0]);
                 const float base = qg == 0 ? 1.0f : qg == 1 ? P : qg == 2 ? R : R * P;
                 float bh[4], kh[4];
-                float *pAs = sA + Ly::oAs + rowbase, *pRs = sA + Ly::oRs + rowbase;
+                float *pAs = sA + Ly::oAs + rowbase, *pRs = sV + Ly::oRs + rowbase;
 #pragma unroll
                 for (int tt = 0; tt < 4; ++tt) {
                     const float gprev = tt == 0 ? base : base * gl[tt - 1];
@@ -545,12 +567,13 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
         for (int it = -4; it < n_chunks + kExtra; ++it) {
             const int c = it + 2;
             if (c >= 0 && c < n_chunks) {
-                const float *sA = ringA + (c % kRA) * Ly::kSlotA;
+                const float *sA = ringA + (c % kRA) * Ly::kStrideA;
+                const float *sV = ringV + (c % kRV) * Ly::kStrideV;
                 float *sG = ringG + (c % kRG) * Ly::kSlotG;
                 floatx4 gab = {0.f, 0.f, 0.f, 0.f}, gp = gab, gqb = gab, gqk = gab;
 #pragma unroll
                 for (int jb = 0; jb < NB; ++jb) {
-                    const floatx4 a4 = ldk(sA + Ly::oAs + li * SA, jb), r4 = ldk(sA + Ly::oRs + li * SA, jb);
+                    const floatx4 a4 = ldk(sA + Ly::oAs + li * SA, jb), r4 = ldk(sV + Ly::oRs + li * SA, jb);
                     // B^[s = li][key of k-step r] from the [key][token] tiles.
                     const int oT = (16 * jb + (half_tile(jb) ? 2 : 4) * g) * kST + li;
                     floatx4 b4 = {0.f, 0.f, 0.f, 0.f}, k4 = b4;
@@ -674,17 +697,21 @@ __global__ void __launch_bounds__((RoleMap<NB, SPLIT>::kWaves) * kWave)
     }
 }
 
-// Heads at or below this many per GPU are split over two workgroups each (the
-// MI355X has 256 CUs; one workgroup per head would leave half of them idle).
-constexpr int kSplitMaxHeads = 128;
+// The nine waves of the N = 64 pair form leave 168 VGPRs, which the fused prep
+// does not fit (it spills); prefills of as many heads run whole heads beside
+// their other parts' kernels anyway.
+constexpr bool op_only(int NB, int VT) { return NB == 4 && VT == 2; }
 
-template <int NB, bool SPLIT, bool HALF>
+template <int NB, int VT, bool HALF>
 void launch_nb_form(const WkvParams &p, int N, bool prep, int units, int per_xcd, hipStream_t stream) {
-    const dim3 grid(per_xcd * kXcds), block(RoleMap<NB, SPLIT>::kWaves * kWave);
-    if (prep)
-        hipLaunchKernelGGL((wkv7_chunk_kernel<NB, true, SPLIT, HALF>), grid, block, 0, stream, p, N, units, per_xcd);
-    else
-        hipLaunchKernelGGL((wkv7_chunk_kernel<NB, false, SPLIT, HALF>), grid, block, 0, stream, p, N, units, per_xcd);
+    const dim3 grid(per_xcd * kXcds), block(RoleMap<NB, VT>::kWaves * kWave);
+    if constexpr (!op_only(NB, VT)) {
+        if (prep) {
+            hipLaunchKernelGGL((wkv7_chunk_kernel<NB, true, (VT > 0), HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((wkv7_chunk_kernel<NB, false, (VT > 0), HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
 }
 
 // Half-padded last key tile (N % 16 == 8) unless YUF_WKV7_HALF=0.
@@ -694,26 +721,37 @@ bool half_tile_form(int N) {
     return !(e && std::strcmp(e, "0") == 0);
 }
 
-template <int NB, bool SPLIT>
-hipError_t launch_nb_split(const WkvParams &p, int N, bool prep, hipStream_t stream) {
-    const int heads = p.B * p.H, units = SPLIT ? 2 * heads : heads;
-    const int per_xcd = (units + kXcds - 1) / kXcds;
-    if (half_tile_form(N)) launch_nb_form<NB, SPLIT, true>(p, N, prep, units, per_xcd, stream);
-    else launch_nb_form<NB, SPLIT, false>(p, N, prep, units, per_xcd, stream);
+template <int NB, int VT>
+hipError_t launch_nb_vt(const WkvParams &p, int N, bool prep, hipStream_t stream) {
+    constexpr int kParts = VT ? (NB + VT - 1) / VT : 1;
+    const int units = p.B * p.H * kParts, per_xcd = (units + kXcds - 1) / kXcds;
+    if (half_tile_form(N)) launch_nb_form<NB, VT, true>(p, N, prep, units, per_xcd, stream);
+    else launch_nb_form<NB, VT, false>(p, N, prep, units, per_xcd, stream);
     return hipGetLastError();
 }
 
-bool split_heads(int heads) {
-    if (const char *e = std::getenv("YUF_WKV7_SPLIT")) return std::strcmp(e, "0") != 0;
-    return heads <= kSplitMaxHeads;
-}
+// Workgroups of a head: one per value tile where all of them run at once (one
+// fits a CU), else two, else one.  A finer split repeats the key-space stages
+// but shortens the busiest SIMD of a chunk; past one round of the 256 CUs it
+// loses.  us for 777 tokens, whole / two / one per tile: N = 64, 48 heads
+// 130 / 104 / 85, 80 heads 129 / 107 / 163, 128 heads 132 / 111 / 171, 192
+// heads 137 / 211 / 245; N = 40, 16 heads 78 / 64.9 / 63.3, 80 heads 80.6 /
+// 68.2 / 67.1, 128 heads 83 / 71 / 126.  YUF_WKV7_SPLIT forces it: 0 whole
+// heads, 1 at least two, 2 two, 4 one per tile.
+constexpr int kCus = 256;
 
 template <int NB>
 hipError_t launch_nb(const WkvParams &p, int N, bool prep, hipStream_t stream) {
-    if constexpr (NB == 2 || NB == 3) {
-        if (split_heads(p.B * p.H)) return launch_nb_split<NB, true>(p, N, prep, stream);
+    if constexpr (NB > 1) {
+        constexpr int kVt2 = (NB + 1) / 2;
+        const int heads = p.B * p.H;
+        const char *e = std::getenv("YUF_WKV7_SPLIT");
+        const int force = e ? std::atoi(e) : -1;
+        const bool two_ok = !(prep && op_only(NB, kVt2));
+        if (force == 4 || (force != 0 && force != 2 && heads * NB <= kCus)) return launch_nb_vt<NB, 1>(p, N, prep, stream);
+        if (two_ok && force != 0 && (force > 0 || heads * 2 <= kCus)) return launch_nb_vt<NB, kVt2>(p, N, prep, stream);
     }
-    return launch_nb_split<NB, false>(p, N, prep, stream);
+    return launch_nb_vt<NB, 0>(p, N, prep, stream);
 }
 
 }  // namespace
