@@ -97,19 +97,15 @@ __global__ void __launch_bounds__(256) ln_shift_kernel(float *__restrict__ x, in
     const int row = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     float *xr = x + (size_t)row * d;
     float *prow = prev_state + (size_t)(slot ? slot[row] : row) * d;
+    // Bounds-checked buffer loads: with a branch around each load the compiler
+    // reused address registers and waited for all loads three times on the way.
     float v[PER], pv[PER], gm[PER], bt[PER], mx[6][PER];
+    const auto rx = make_rsrc(xr, (uint32_t)d * 4u), rpv = make_rsrc(prow, (uint32_t)d * 4u);
+    const auto rg = make_rsrc(gamma, (uint32_t)d * 4u), rb = make_rsrc(beta, (uint32_t)d * 4u);
+    const auto rmx = make_rsrc(mix6, (uint32_t)d * 24u);
     float sum = 0.0f;
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-        const int c = tid + e * 256;
-        const bool ok = c < d;
-        v[e] = ok ? xr[c] : 0.0f;
-        pv[e] = ok ? prow[c] : 0.0f;
-        gm[e] = ok ? gamma[c] : 0.0f;
-        bt[e] = ok ? beta[c] : 0.0f;
-#pragma unroll
-        for (int q = 0; q < 6; ++q) mx[q][e] = ok ? mix6[q * d + c] : 0.0f;
-    }
+    for (int e = 0; e < PER; ++e) v[e] = buf_load(rx, (uint32_t)(tid + e * 256) * 4u);
     // Pending K-split partial sums of the previous product (h += P0 + P1 + ...,
     // in order): loaded with the row (unused parts read as zero outside the
     // descriptor), the row is completed and written back before it is normed.
@@ -123,6 +119,16 @@ __global__ void __launch_bounds__(256) ln_shift_kernel(float *__restrict__ x, in
             const int c = tid + e * 256;
             pp[q][e] = buf_load(rpart, q < nparts && c < d ? (uint32_t)((size_t)q * part_stride + c) * 4u : kBufferOob);
         }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        const int c = tid + e * 256;
+        const uint32_t off = (uint32_t)c * 4u;
+        pv[e] = buf_load(rpv, off);
+        gm[e] = buf_load(rg, off);
+        bt[e] = buf_load(rb, off);
+#pragma unroll
+        for (int q = 0; q < 6; ++q) mx[q][e] = buf_load(rmx, c < d ? off + (uint32_t)(q * d) * 4u : kBufferOob);
+    }
 #pragma unroll
     for (int q = 0; q < kMaxParts; ++q)
         if (q < nparts) {

@@ -1273,35 +1273,47 @@ __global__ void __launch_bounds__(kDecThreads) gemm_decode_kernel(DecodeGroup g)
                               PRO == 2 ? (p.a_tiled ? (uint32_t)((size_t)RT * p.ldg * 4)
                                                     : (uint32_t)(((size_t)(rows - 1) * p.ldg + p.K) * 4))
                                        : 0u);
+    // Both layouts of W (tiled or row-major) and of A and the gate (tile_index or
+    // row-major) are a row offset plus k / tile * step + k % tile, so one load
+    // serves both.  (With the layouts as the two arms of a condition each A load
+    // became a branch, whose second arm waited for every load before it: five
+    // memory round trips in a row at K = 640.)
+    uint32_t wrow[NT], arow[MI], grow[PRO == 2 ? MI : 1];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const uint32_t wr = w_row0 + 32 * t + li;
+        wrow[t] = (int)wr >= p.N ? kBufferOob : tiled ? (wr >> 4) * (uint32_t)p.wt_ld + (wr & 15) * KS : wr * (uint32_t)p.ldw;
+    }
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        arow[i] = p.a_tiled ? (uint32_t)(16 * p.lda * i + li * 16) : (uint32_t)((16 * i + li) * p.lda);
+        if constexpr (PRO == 2) grow[i] = p.a_tiled ? (uint32_t)(16 * p.ldg * i + li * 16) : (uint32_t)((16 * i + li) * p.ldg);
+    }
+    const uint32_t wstep = tiled ? 16 * KS : KS, astep = p.a_tiled ? 256 : 16;
     auto load_w = [&](int s, int k0) __attribute__((always_inline)) {
         const int k = k0 + KS * s + RL * g4;
         const bool kin = k < k_end;  // K % RL == 0 on this path
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int wr = w_row0 + 32 * t + li;
-            const size_t e = tiled ? (size_t)(wr >> 4) * p.wt_ld + (size_t)(k / KS) * (16 * KS) + (wr & 15) * KS + (k % KS)
-                                   : (size_t)wr * p.ldw + k;
-            b[s][t] = load4(rw, (kin && wr < p.N) ? (uint32_t)e * (WB ? 2u : 4u) : kBufferOob);
+            const uint32_t e = wrow[t] + (uint32_t)(k / KS) * wstep + (uint32_t)(k % KS);
+            b[s][t] = load4(rw, kin && wrow[t] != kBufferOob ? e * (WB ? 2u : 4u) : kBufferOob);
         }
     };
+    auto aoff = [&](int k) __attribute__((always_inline)) { return (uint32_t)(k >> 4) * astep + (uint32_t)(k & 15); };
     auto load_a = [&](int s, int k0) __attribute__((always_inline)) {
         const int k = k0 + KS * s + RL * g4;
-        const bool kin = k < k_end;
+        const uint32_t oob = k < k_end ? 0u : kBufferOob;
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
             for (int hh = 0; hh < AH; ++hh)
-                a[s][i][hh] = load4(ra, kin ? (uint32_t)(p.a_tiled ? tile_index(16 * i + li, k + 4 * hh, p.lda)
-                                                                   : (size_t)(16 * i + li) * p.lda + k + 4 * hh) * 4u
-                                            : kBufferOob);
+                a[s][i][hh] = load4(ra, ((arow[i] + aoff(k + 4 * hh)) * 4u) | oob);
         if constexpr (PRO == 2) {
 #pragma unroll
             for (int i = 0; i < MI; ++i)
 #pragma unroll
                 for (int hh = 0; hh < AH; ++hh)
-                    gt[s][i][hh] = load4(rt, kin ? (uint32_t)(p.a_tiled ? tile_index(16 * i + li, k + 4 * hh, p.ldg)
-                                                                        : (size_t)(16 * i + li) * p.ldg + k + 4 * hh) * 4u
-                                                 : kBufferOob);
+                    gt[s][i][hh] = load4(rt, ((grow[i] + aoff(k + 4 * hh)) * 4u) | oob);
         }
     };
     // Issue order: with a prologue, all A (and gate) loads of the round first,
@@ -1337,6 +1349,22 @@ __global__ void __launch_bounds__(kDecThreads) gemm_decode_kernel(DecodeGroup g)
         for (int s = 0; s < S; ++s) load_w(s, k_begin);
     } else {
         load_round(k_begin);
+    }
+    // The epilogue's bias and residual, in flight behind the operands: read
+    // after the reduction they cost a memory round trip of their own.
+    constexpr int kEp = (RT * 16 + kDecThreads - 1) / kDecThreads;  // elements per thread
+    float bias[NT == 1 ? kEp : 1], res[NT == 1 ? kEp : 1];
+    if constexpr (NT == 1) {
+        const auto rb = make_rsrc(p.bias, p.bias ? (uint32_t)p.N * 4u : 0u);
+        const auto rr = make_rsrc(p.residual ? p.residual + (size_t)row0 * p.ldr : nullptr,
+                                  p.residual ? (uint32_t)(((size_t)(rows - 1) * p.ldr + p.N) * 4) : 0u);
+#pragma unroll
+        for (int e = 0; e < kEp; ++e) {
+            const int q = tid + e * kDecThreads, rl = q >> 4, col = w_row0 + (q & 15);
+            const bool ok = rl < rows && col < p.N;
+            bias[e] = buf_load(rb, ok ? (uint32_t)col * 4u : kBufferOob);
+            res[e] = buf_load(rr, ok ? (uint32_t)(rl * p.ldr + col) * 4u : kBufferOob);
+        }
     }
 
     float mean[MI], rstd[MI];
@@ -1488,8 +1516,9 @@ __global__ void __launch_bounds__(kDecThreads) gemm_decode_kernel(DecodeGroup g)
 #pragma unroll
             for (int r = 0; r < 4; ++r) red[wave][t][(16 * i + 4 * g4 + r) * 17 + li] = acc[t][i][r];
     lds_barrier();
-    for (int q = tid; q < RT * 16; q += kDecThreads) {
-        const int rl = q >> 4, c = q & 15;
+#pragma unroll
+    for (int e = 0; e < kEp; ++e) {
+        const int q = tid + e * kDecThreads, rl = q >> 4, c = q & 15;
         if (rl >= rows) continue;
         const int row = row0 + rl;
         float x[NT];
@@ -1506,8 +1535,8 @@ __global__ void __launch_bounds__(kDecThreads) gemm_decode_kernel(DecodeGroup g)
         } else {
             const int col = w_row0 + c;
             if (col < p.N) {
-                float y = apply_act(x[0] + (p.bias ? p.bias[col] : 0.0f), p.act);
-                if (p.residual) y += p.residual[(size_t)row * p.ldr + col];
+                float y = apply_act(x[0] + bias[e], p.act);
+                if (p.residual) y += res[e];
                 p.C[(size_t)row * p.ldc + col] = y;
             }
         }
@@ -1690,7 +1719,8 @@ __global__ void __launch_bounds__(kDecThreads) rosa_out_decode_kernel(RosaOutPar
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g4 = lane >> 4, li = lane & 15;
     const bool rv = li < rows;
-    const int slot = rv ? (p.slot ? p.slot[row0 + li] : row0 + li) : 0;
+    const auto rs = make_rsrc(p.slot ? p.slot + row0 : nullptr, p.slot ? (uint32_t)rows * 4u : 0u);
+    const int listed = __float_as_int(buf_load(rs, (uint32_t)li * 4u));
     const int D = p.D, kw = wave * 16 * S;
     const auto rm = make_rsrc(p.mem, (uint32_t)((size_t)p.mem_rows * D * 4));
     const auto rp = make_rsrc(p.pre + (size_t)row0 * p.ld_pre, (uint32_t)(((size_t)(rows - 1) * p.ld_pre + 3 * D) * 4));
@@ -1708,13 +1738,25 @@ __global__ void __launch_bounds__(kDecThreads) rosa_out_decode_kernel(RosaOutPar
         const int k = kw + 16 * s + 4 * g4;
         const size_t we = tiled ? (size_t)slice * p.wt_ld + (size_t)(k >> 4) * 256 + li * 16 + (k & 15) : (size_t)wr * D + k;
         b[s] = load4(rw, wr < p.N ? (uint32_t)we * 4u : kBufferOob);
-        m[s] = load4(rm, rv ? (uint32_t)((size_t)slot * D + k) * 4u : kBufferOob);
         e[s] = load4(rp, rv ? (uint32_t)((size_t)li * p.ld_pre + k) * 4u : kBufferOob);
         gw[s] = load4(rp, rv ? (uint32_t)((size_t)li * p.ld_pre + D + k) * 4u : kBufferOob);
         rr[s] = load4(rp, rv ? (uint32_t)((size_t)li * p.ld_pre + 2 * D + k) * 4u : kBufferOob);
         uu[s] = load4(ru, (uint32_t)k * 4u);
         ll[s] = load4(rl, (uint32_t)k * 4u);
     }
+    // Last, as its address waits for the slot.
+    const int slot = p.slot ? listed : row0 + li;
+#pragma unroll
+    for (int s = 0; s < S; ++s)
+        m[s] = load4(rm, ((uint32_t)(slot * D + kw + 16 * s + 4 * g4) * 4u) | (rv ? 0u : kBufferOob));
+    // The epilogue's bias and residual, in flight behind the operands.
+    const int orow = tid >> 4, ocol = slice * 16 + (tid & 15);
+    const bool out_ok = orow < rows && ocol < p.N;
+    const auto rbias = make_rsrc(p.bias, p.bias ? (uint32_t)p.N * 4u : 0u);
+    const auto rres = make_rsrc(p.residual ? p.residual + (size_t)row0 * p.ldr : nullptr,
+                                p.residual ? (uint32_t)(((size_t)(rows - 1) * p.ldr + p.N) * 4) : 0u);
+    const float bias = buf_load(rbias, out_ok ? (uint32_t)ocol * 4u : kBufferOob);
+    const float res = buf_load(rres, out_ok ? (uint32_t)(orow * p.ldr + ocol) * 4u : kBufferOob);
     // Gates (the single-token kernel's expressions): e <- tanh(e) sigmoid(write),
     // rr <- sigmoid(read_raw); first projection u.m.
     double f = 0.0;
@@ -1730,6 +1772,12 @@ __global__ void __launch_bounds__(kDecThreads) rosa_out_decode_kernel(RosaOutPar
     f = rows_sum_f64(f);
     if (g4 == 0) pd[0][wave][li] = f;
     lds_barrier();
+    // Every wave holds its old memory values (f needed them): count this
+    // workgroup now, so the atomic's round trip runs beside the product; the
+    // tile's last one, which wraps the counter to 0, writes the new rows.
+    const unsigned others = units / mtiles - 1;
+    unsigned count = 0;
+    if (tid == 0) count = atomicInc(reinterpret_cast<unsigned *>(&p.counter[mt]), others);
     double t = 0.0;
 #pragma unroll
     for (int w = 0; w < kDecWaves; ++w) t += pd[0][w][li];
@@ -1761,23 +1809,16 @@ __global__ void __launch_bounds__(kDecThreads) rosa_out_decode_kernel(RosaOutPar
     // Register r of lane l: row 4 (l / 16) + r, column l % 16.
 #pragma unroll
     for (int r = 0; r < 4; ++r) red[wave][(4 * g4 + r) * 17 + li] = acc[r];
+    if (tid == 0) last = count == others;
     lds_barrier();
-    if (tid < 256) {
-        const int rl = tid >> 4, c = tid & 15, col = slice * 16 + c;
-        if (rl < rows && col < p.N) {
-            float x = 0.0f;
+    if (tid < 256 && out_ok) {
+        float x = 0.0f;
 #pragma unroll
-            for (int w = 0; w < kDecWaves; ++w) x += red[w][rl * 17 + c];
-            const int row = row0 + rl;
-            if (p.bias) x += p.bias[col];
-            if (p.residual) x += p.residual[(size_t)row * p.ldr + col];
-            p.C[(size_t)row * p.ldc + col] = x;
-        }
+        for (int w = 0; w < kDecWaves; ++w) x += red[w][orow * 17 + (tid & 15)];
+        if (p.bias) x += bias;
+        if (p.residual) x += res;
+        p.C[(size_t)(row0 + orow) * p.ldc + ocol] = x;
     }
-    // Every wave has consumed its old memory values (p1 needed them): count
-    // this workgroup; the tile's last one writes the new rows.
-    if (tid == 0) last = atomicAdd(&p.counter[mt], 1) == units / mtiles - 1;
-    lds_barrier();
     if (last) {
         if (rv) {
 #pragma unroll
@@ -1787,7 +1828,6 @@ __global__ void __launch_bounds__(kDecThreads) rosa_out_decode_kernel(RosaOutPar
                                                        (uint32_t)((size_t)slot * D + k) * 4u, 0, 0);
             }
         }
-        if (tid == 0) atomicExch(&p.counter[mt], 0);
     }
 }
 

@@ -318,10 +318,10 @@ __global__ void __launch_bounds__(kWave) wkv7_scan_kernel(WkvParams p, int waves
 // LR (model decode path): the second low-rank stage runs here instead of as a
 // GEMM -- w, alpha and the output gate g of the head's N channels are dot
 // products of the stream's rank-L rows with the head's N x L slices of w2t,
-// a2t, g2t, staged once per workgroup in LDS and shared by its SPW streams.
+// a2t, g2t, read once per workgroup and shared by its SPW streams.
 constexpr int kStepThreads = 256;
 constexpr int kStepLrSpw = 4;       // streams per workgroup of the LR form
-constexpr int kStepLrMaxL = 128;  // an LDS weight row holds kStepLrMaxL + 2 floats (even / odd lanes on distinct banks)
+constexpr int kStepLrMaxL = 128;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 template <int N, bool PREP, int SPW, bool LR>
@@ -330,16 +330,14 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
     constexpr int Q = N * N / 4;                                 // float4 of the state
     constexpr int QM = (Q + kStepThreads - 1) / kStepThreads;   // per thread
     constexpr int RQ = N / 4;                                    // float4 per row
-    constexpr int LP = kStepLrMaxL + 2;                          // padded LDS row of a weight slice
     __shared__ __attribute__((aligned(16))) float vec[SPW][6][N];  // a, b, k^, d, r, v
     __shared__ float part[SPW][Q];                                 // per-float4 partial row sums
     __shared__ float rowv[SPW][N];                                 // S a, then y
-    __shared__ float red[SPW][kStepThreads / 64];
-    __shared__ float wl[LR ? 3 * N : 1][LR ? LP : 1];              // w2t | a2t | g2t rows of the head
-    __shared__ float lrs[LR ? SPW : 1][LR ? 3 : 1][LR ? kStepLrMaxL : 1];
+    __shared__ float red[N > 64 ? SPW : 1][kStepThreads / 64];
+    __shared__ __attribute__((aligned(16))) float lrs[LR ? SPW : 1][LR ? 3 : 1][LR ? kStepLrMaxL : 1];
     __shared__ float lrv[LR ? SPW : 1][2][LR ? N : 1];             // w, alpha
 
-    const int sub = threadIdx.x / kStepThreads, tid = threadIdx.x % kStepThreads;
+    const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x / kStepThreads), tid = threadIdx.x % kStepThreads;
     const int lane = tid & 63, wave = tid >> 6;
     const int h = blockIdx.x % p.H, bb = (blockIdx.x / p.H) * SPW + sub;
     const bool live = bb < p.B;  // idle streams of the last workgroup still meet every barrier
@@ -347,15 +345,18 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
     const size_t state_off = ((size_t)slot * p.H + h) * N * N;
     const size_t base = ((size_t)(live ? bb : 0) * p.H + h) * N;  // token (bb, 0)
 
-    // All global loads first: the state's float4s, then one column / row per thread.
+    // All global loads first: one column / row per thread, then the state's
+    // float4s, whose address waits for the slot.
     const auto rs = make_rsrc(live && p.state_in ? p.state_in + state_off : nullptr,
                               live && p.state_in ? N * N * 4 : 0u);
     float4 sq[QM];
+    auto load_state = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int m = 0; m < QM; ++m) {
-        const int q = tid + m * kStepThreads;
-        sq[m] = buf_load4(rs, q < Q ? (uint32_t)q * 16u : kBufferOob);
-    }
+        for (int m = 0; m < QM; ++m) {
+            const int q = tid + m * kStepThreads;
+            sq[m] = buf_load4(rs, q < Q ? (uint32_t)q * 16u : kBufferOob);
+        }
+    };
     const bool col = tid < N;
     const uint32_t off = col && live ? (uint32_t)tid * 4u : kBufferOob;
     const float rv = buf_load(make_rsrc(p.r + base, N * 4), off);
@@ -366,32 +367,38 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
     }
     float kv = buf_load(make_rsrc(p.k + base, N * 4), off);
     const float vv = buf_load(make_rsrc(p.v + base, N * 4), off);
-    float bv = 0.0f, kk = 0.0f, ka = 0.0f;
+    float bv = 0.0f, kk = 0.0f, ka = 0.0f, ksq = 0.0f;
     if constexpr (PREP) {
         kk = buf_load(make_rsrc(p.k_k + h * N, N * 4), off);
         ka = buf_load(make_rsrc(p.k_a + h * N, N * 4), off);
     } else {
         bv = buf_load(make_rsrc(p.b + base, N * 4), off);
     }
+    if constexpr (!LR) load_state();
     if constexpr (LR) {
-        // Stage the head's weight rows (3 N rows of L, contiguous N x L blocks)
-        // and the streams' rank-L rows: every load is issued before the first
-        // LDS write, so staging costs one memory latency.
+        // Dot dq = m N + c of the head runs on eight lanes for all of the
+        // workgroup's streams: a lane's weights, 16-byte runs 32 k apart, go from
+        // memory to registers, and only the streams' rank-L rows are staged.
+        // Every load is issued before the first LDS write, so this costs one
+        // memory latency.  (N % 8 == 0: m is uniform over a wave.)
         constexpr int kT = kStepThreads * SPW;
-        constexpr int kW4 = (N * kStepLrMaxL / 4 + kT - 1) / kT;  // float4 per thread and matrix
+        constexpr int kDl = 8, kI = kStepLrMaxL / (4 * kDl), kP = (3 * N * kDl + kT - 1) / kT;
         constexpr int kL1 = (SPW * 3 * kStepLrMaxL + kT - 1) / kT;
-        const int L = p.L, nl4 = N * L / 4, flat = threadIdx.x;
-        float4 wreg[3][kW4];
+        static_assert(N % 8 == 0 && SPW <= kDl, "dot layout");
+        const int L = p.L, flat = threadIdx.x, dl = flat % kDl;
+        float4 wreg[kP][kI];
 #pragma unroll
-        for (int m = 0; m < 3; ++m) {
+        for (int ps = 0; ps < kP; ++ps) {
+            const int dq = (flat + ps * kT) / kDl, m = __builtin_amdgcn_readfirstlane(dq / N), c = dq - m * N;
             const float *src = m == 0 ? p.w2t : (m == 1 ? p.a2t : p.g2t);
-            const auto rw = make_rsrc(src + (size_t)h * N * L, (uint32_t)(N * L * 4));
+            const auto rw = make_rsrc(src + (size_t)h * N * L, m < 3 ? (uint32_t)(N * L * 4) : 0u);
 #pragma unroll
-            for (int i = 0; i < kW4; ++i) {
-                const int e4 = flat + i * kT;
-                wreg[m][i] = buf_load4(rw, e4 < nl4 ? (uint32_t)e4 * 16u : kBufferOob);
+            for (int i = 0; i < kI; ++i) {
+                const int j = 4 * (dl + kDl * i);
+                wreg[ps][i] = buf_load4(rw, j < L ? (uint32_t)(c * L + j) * 4u : kBufferOob);
             }
         }
+        const auto rlr = make_rsrc(p.lr, (uint32_t)((2 * p.lr_plane + (size_t)p.B * L) * 4));
         float lreg[kL1];
 #pragma unroll
         for (int i = 0; i < kL1; ++i) {
@@ -399,50 +406,54 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
             const int sb = e / (3 * L), rem = e - sb * 3 * L, m = rem / L, j = rem - m * L;
             const int b2 = (blockIdx.x / p.H) * SPW + sb;
             const bool ok = sb < SPW && b2 < p.B;
-            lreg[i] = ok ? p.lr[m * p.lr_plane + (size_t)b2 * L + j] : 0.0f;
+            lreg[i] = buf_load(rlr, (((uint32_t)m * (uint32_t)p.lr_plane + (uint32_t)(b2 * L + j)) * 4u) | (ok ? 0u : kBufferOob));
         }
-        const float w0c = col ? p.w0[h * N + tid] : 0.0f, a0c = col ? p.a0[h * N + tid] : 0.0f;
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-#pragma unroll
-            for (int i = 0; i < kW4; ++i) {
-                const int e4 = flat + i * kT;
-                if (e4 < nl4) {
-                    const int c = (4 * e4) / L, j = 4 * e4 - c * L;  // L % 8 == 0
-                    float *dst = &wl[m * N + c][j];
-                    dst[0] = wreg[m][i].x; dst[1] = wreg[m][i].y; dst[2] = wreg[m][i].z; dst[3] = wreg[m][i].w;
-                }
-            }
+        const float w0c = buf_load(make_rsrc(p.w0 + h * N, N * 4), col ? (uint32_t)tid * 4u : kBufferOob);
+        const float a0c = buf_load(make_rsrc(p.a0 + h * N, N * 4), col ? (uint32_t)tid * 4u : kBufferOob);
+        load_state();
 #pragma unroll
         for (int i = 0; i < kL1; ++i) {
             const int e = flat + i * kT;
             const int sb = e / (3 * L), rem = e - sb * 3 * L, m = rem / L, j = rem - m * L;
             if (sb < SPW) lrs[sb][m][j] = lreg[i];
         }
+        ksq = wave_sum((kv * kk) * (kv * kk));
         lds_barrier();
-        // One dot per thread (PAIR = false) or per lane pair, the even and odd
-        // j of a dot on lanes 2q and 2q + 1, summed through a DPP swap.
-        constexpr bool PAIR = 6 * N <= kStepThreads;
-        constexpr int TPD = PAIR ? 2 : 1;
-        if (tid < 3 * N * TPD) {
-            const int dq = tid / TPD, hj = tid % TPD, m = dq / N, c = dq - m * N;
-            const float *wrow = &wl[m * N + c][hj];
-            const float *lrow = &lrs[sub][m][hj];
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll 4
-            for (int i = 0; i < L / TPD; i += 4)  // L % 8 == 0
 #pragma unroll
-                for (int t = 0; t < 4; ++t) acc[t] = fmaf(lrow[TPD * (i + t)], wrow[TPD * (i + t)], acc[t]);
-            float dot = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-            if constexpr (PAIR) dot += dpp_move<dpp::kQuadXor1>(dot);
-            if (hj == 0) {
-                if (m == 2) {
-                    if (live)
-                        p.g_out[p.tiled_out ? tile_index(bb, h * N + c, p.H * N) : (size_t)bb * p.H * N + h * N + c] =
-                            1.0f / (1.0f + expf(-dot));
-                } else {
-                    lrv[sub][m][c] = dot;
+        for (int ps = 0; ps < kP; ++ps) {
+            const int dq = (flat + ps * kT) / kDl, m = __builtin_amdgcn_readfirstlane(dq / N), c = dq - m * N;
+            if (m >= 3) break;  // uniform over the wave
+            float acc[SPW];
+#pragma unroll
+            for (int st = 0; st < SPW; ++st) acc[st] = 0.0f;
+#pragma unroll
+            for (int i = 0; i < kI; ++i) {
+                const int j = 4 * (dl + kDl * i);
+                if (j < L) {
+#pragma unroll
+                    for (int st = 0; st < SPW; ++st) {
+                        const float4 l4 = *reinterpret_cast<const float4 *>(&lrs[st][m][j]);
+                        acc[st] = fmaf(l4.x, wreg[ps][i].x, acc[st]);
+                        acc[st] = fmaf(l4.y, wreg[ps][i].y, acc[st]);
+                        acc[st] = fmaf(l4.z, wreg[ps][i].z, acc[st]);
+                        acc[st] = fmaf(l4.w, wreg[ps][i].w, acc[st]);
+                    }
                 }
+            }
+            // Lane st of the eight keeps stream st's dot.
+            float dot = 0.0f;
+#pragma unroll
+            for (int st = 0; st < SPW; ++st) {
+                const float sum = group_sum<kDl>(acc[st]);
+                dot = dl == st ? sum : dot;
+            }
+            if (dl < SPW) {
+                const int b2 = (blockIdx.x / p.H) * SPW + dl;
+                if (m < 2)
+                    lrv[dl][m][c] = dot;
+                else if (b2 < p.B)
+                    p.g_out[p.tiled_out ? tile_index(b2, h * N + c, p.H * N) : (size_t)b2 * p.H * N + h * N + c] =
+                        1.0f / (1.0f + expf(-dot));
             }
         }
         lds_barrier();
@@ -452,14 +463,18 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
         }
     }
     if constexpr (PREP) {
-        // kappa = normalize(k * k_k) over the head (F.normalize, eps 1e-12).
+        // kappa = normalize(k * k_k) over the head (F.normalize, eps 1e-12); a
+        // head of up to 64 columns lies in one wave.
         const float x = kv * kk;
-        const float ws = wave_sum(x * x);
-        if (lane == 0) red[sub][wave] = ws;
-        lds_barrier();
-        float sq2 = 0.0f;
+        if constexpr (!LR) ksq = wave_sum(x * x);
+        float sq2 = ksq;
+        if constexpr (N > 64) {
+            if (lane == 0) red[sub][wave] = ksq;
+            lds_barrier();
+            sq2 = 0.0f;
 #pragma unroll
-        for (int w = 0; w < (N + 63) / 64; ++w) sq2 += red[sub][w];
+            for (int w = 0; w < (N + 63) / 64; ++w) sq2 += red[sub][w];
+        }
         const float inv = 1.0f / fmaxf(sqrtf(sq2), 1e-12f);
         const float kap = x * inv, alpha = av;
         av = -kap;
