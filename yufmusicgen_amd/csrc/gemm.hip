@@ -1277,7 +1277,8 @@ __global__ void __launch_bounds__(kDecThreads) gemm_decode_kernel(DecodeGroup g)
     // row-major) are a row offset plus k / tile * step + k % tile, so one load
     // serves both.  (With the layouts as the two arms of a condition each A load
     // became a branch, whose second arm waited for every load before it: five
-    // memory round trips in a row at K = 640.)
+    // memory round trips in a row at K = 640.  640 x 640 with LN and gate, one
+    // row, 7.5 -> 6.6 us.)
     uint32_t wrow[NT], arow[MI], grow[PRO == 2 ? MI : 1];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {

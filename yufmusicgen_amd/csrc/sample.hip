@@ -435,7 +435,8 @@ __global__ void __launch_bounds__(NTH) sample_kernel(SampleParams p) {
 //      8-bit digits, four passes (a pass whose digit is the same for every
 //      value is skipped).  The sort is bound by vector instructions of the one
 //      CU, about in proportion to digit passes: a wave owns R x 64 consecutive
-//      positions, eight ballots rank a round's lanes among their equal digits,
+//      positions (64 rows of 20480: 119 us, 171 with eight 4-bit
+//      passes), eight ballots rank a round's lanes among their equal digits,
 //      a running count per (digit, wave) in LDS carries the rank over the
 //      rounds, and what it ends at, scanned in (digit, wave) order, places the
 //      elements;
