@@ -236,6 +236,34 @@ def test_full_vocab_sort_edges(vocab):
         np.testing.assert_array_equal(tokens.cpu().numpy(), np.array(expect), err_msg=f"step {step}")
 
 
+@pytest.mark.parametrize("vocab", [1024, 20480])
+def test_full_vocab_sort_when_lane_zero_sees_one_digit(vocab):
+    """Whether a sort pass can be skipped is a vote of the workgroup: rows whose
+    ids 0 mod 64 (lane 0 of every wave, in every round) share the digit of a
+    pass and whose other ids do not, for each of the four 8-bit digits alone and
+    for two plain values.  The host's tokens."""
+    print(f"sampler digit vote V={vocab}", flush=True)
+    rng = np.random.default_rng(31 + vocab)
+    lane0 = np.arange(vocab) % 64 == 0
+    rows = [np.where(lane0, 1.0, -2.0).astype(np.float32)]
+    for byte, digits in enumerate((np.arange(256), np.arange(256), np.arange(0x80, 0xE0), [0x3E, 0x3F, 0xBE, 0xBF])):
+        bits = np.full(vocab, 0x3FC04020, dtype=np.uint32)
+        pick = rng.choice(np.asarray(digits, dtype=np.uint32), vocab) << np.uint32(8 * byte)
+        mixed = (bits & np.uint32(~(0xFF << (8 * byte)) & 0xFFFFFFFF)) | pick
+        rows.append(np.where(lane0, bits, mixed).astype(np.uint32).view(np.float32))
+    x = np.stack(rows)
+    logits = torch.from_numpy(x).cuda()
+    tokens = torch.empty(len(rows), dtype=torch.int32, device="cuda")
+    host = [Mt19937(60 + s) for s in range(len(rows))]
+    dev = [g.copy() for g in host]
+    for step in range(3):
+        q, _ = _exact_draws(dev, vocab, vocab)
+        sample_device_masked(logits, tokens, 1.0, 0.9, 0, exp_draws=q)
+        torch.cuda.synchronize()
+        expect = [sample_token(x[s], 1.0, 0.9, host[s], top_k=0) for s in range(len(rows))]
+        np.testing.assert_array_equal(tokens.cpu().numpy(), np.array(expect), err_msg=f"step {step}")
+
+
 def test_full_vocab_counter_mode_stays_in_the_nucleus():
     """Counter draws (no host work): every token lies in the host's nucleus of
     the masked row, and a near-flat row spreads over many ids."""

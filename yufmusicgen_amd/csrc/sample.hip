@@ -607,8 +607,10 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(SampleParams 
                 one_digit &= ((kr[r] >> shift) & 255u) == d0;
             }
         // A digit that every element shares leaves the order unchanged.
-        if (lane == 0) sh_int2[wave] = 1;
-        if (!one_digit) sh_int2[wave] = 0;
+        // (Voted in the wave and stored by one lane: lanes that store different
+        // values to one word have no defined outcome.)
+        const int wave_one_digit = __all(one_digit);
+        if (lane == 0) sh_int2[wave] = wave_one_digit;
         reinterpret_cast<uint2 *>(scnt32)[tid] = make_uint2(0u, 0u);
         __syncthreads();
         int same_digit = 1;
