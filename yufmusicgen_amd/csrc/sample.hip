@@ -543,7 +543,7 @@ __global__ void __launch_bounds__(kFullThreads) sample_full_kernel(SampleParams 
     __shared__ uint16_t sidx[kFullMaxV];  // token ids; kDropBit once cut by top-p
     // Digit counts, then their offsets, per (digit, wave); before the sort, the
     // blocked-id bitmap of the generation mask.
-    __shared__ uint32_t scnt32[kFullDigits * kFullWaves / 2];
+    __shared__ __attribute__((aligned(8))) uint32_t scnt32[kFullDigits * kFullWaves / 2];  // cleared and scanned as uint2
     __shared__ uint64_t sh_u64[kFullWaves];
     __shared__ double sh_f64[kFullWaves];
     __shared__ int sh_int[kFullWaves], sh_int2[kFullWaves];
