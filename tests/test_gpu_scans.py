@@ -261,3 +261,97 @@ def test_rosa_segments(dim, steps):
         re, me = orosa.rosa_scan(*t64, gated=gated)
         np.testing.assert_allclose(out.cpu().numpy(), re.numpy(), rtol=RTOL, atol=ATOL)
         np.testing.assert_allclose(mem.cpu().numpy(), me.numpy(), rtol=RTOL, atol=ATOL)
+
+
+def _rosa_call(args, mem, out, gated, stream):
+    from yufmusicgen_amd._lib import check, lib
+
+    cand, write, read_raw, decay, u = args
+    batch, steps, dim = cand.shape
+    check(lib().yuf_rosa_scan_f32(batch, steps, dim, cand.data_ptr(), write.data_ptr(),
+                                  read_raw.data_ptr() if gated else None, decay.data_ptr(), u.data_ptr(),
+                                  mem.data_ptr(), mem.data_ptr(), out.data_ptr(), stream))
+
+
+@pytest.mark.parametrize("steps", [640, 1100])
+def test_rosa_operator_under_capture(steps):
+    """The operator captured into a graph, on a stream that has a scratch buffer
+    and on one that has none, and replayed between eager calls on the capturing
+    stream that outgrow every buffer (ragged and whole lengths): each replay
+    gives the eager call's result -- bit for bit at a multiple of 64, where both
+    run in segments, and to the tolerance of the scans at a ragged length, which
+    a graph runs as one segment."""
+    dim = 128
+    args = [_dev(x) for x in rosa_inputs(77, 2, steps, dim)]
+    m0 = _dev(np.random.default_rng(3).standard_normal((2, dim)).astype(np.float32))
+    torch.cuda.synchronize()
+    for warm in (True, False):
+        print(f"rosa capture T={steps} warm={warm}", flush=True)
+        st = torch.cuda.Stream()
+        mem, out = m0.clone(), torch.full((2, steps, dim), float("nan"), device="cuda")
+        torch.cuda.synchronize()
+        with torch.cuda.stream(torch.cuda.current_stream() if not warm else st):
+            _rosa_call(args, mem, out, True, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        want, want_mem = out.clone(), mem.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            _rosa_call(args, mem, out, True, st.cuda_stream)
+        for i, (batch, length) in enumerate(((2, 1111), (4, 2048), (8, 4161))):
+            big = [_dev(x) for x in rosa_inputs(i, batch, length, dim)]
+            big_mem, big_out = torch.zeros(batch, dim, device="cuda"), torch.empty(batch, length, dim, device="cuda")
+            mem.copy_(m0)
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            _rosa_call(big, big_mem, big_out, True, st.cuda_stream)
+            with torch.cuda.stream(st):
+                graph.replay()
+            torch.cuda.synchronize()
+            if steps % 64 == 0:
+                assert torch.equal(out, want) and torch.equal(mem, want_mem), i
+            else:
+                torch.testing.assert_close(out, want, rtol=RTOL, atol=ATOL)
+                torch.testing.assert_close(mem, want_mem, rtol=RTOL, atol=ATOL)
+            assert torch.isfinite(big_out).all()
+
+
+@pytest.mark.parametrize("shared", ["stream", "per_thread_default"])
+def test_rosa_operator_from_several_threads(shared):
+    """Two host threads call the operator at lengths that need scratch, on one
+    stream and on the per-thread default stream (one handle, a stream per
+    thread): every call gives the result of the same call alone."""
+    import threading
+
+    print(f"rosa threads {shared}", flush=True)
+    dim = 128
+    jobs = []
+    for seed, steps in ((5, 1100), (6, 705)):
+        args = [_dev(x) for x in rosa_inputs(seed, 2, steps, dim)]
+        mem, out = torch.zeros(2, dim, device="cuda"), torch.empty(2, steps, dim, device="cuda")
+        torch.cuda.synchronize()
+        _rosa_call(args, mem, out, True, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        reps = [(torch.zeros(2, dim, device="cuda"), torch.empty(2, steps, dim, device="cuda")) for _ in range(40)]
+        jobs.append((args, mem, out, reps))
+    st = torch.cuda.Stream()
+    handle = st.cuda_stream if shared == "stream" else 2  # hipStreamPerThread
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(args, reps):
+        try:
+            for mem, out in reps:
+                _rosa_call(args, mem, out, True, handle)
+        except Exception as exc:  # noqa: BLE001 - reported below
+            errors.append(exc)
+
+    threads = [threading.Thread(target=work, args=(args, reps)) for args, _, _, reps in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for _, mem, out, reps in jobs:
+        for i, (m, o) in enumerate(reps):
+            assert torch.equal(m, mem) and torch.equal(o, out), i

@@ -36,10 +36,13 @@
 #include "common.h"
 #include "kernels.h"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <thread>
+#include <tuple>
 #include <utility>
 
 namespace yuf {
@@ -1041,32 +1044,43 @@ hipError_t launch_rosa_segmented(const RosaParams &p, const float *AL, float *sc
 }
 
 namespace {
-// Operator path: scratch of the segmented scan, one growing buffer per (device, stream) kept for the life of the process (a
-// launch on a stream only ever waits on that stream's earlier work).
+// Operator path: scratch of the segmented scan, one growing buffer per (device,
+// stream) kept for the life of the process.  A stream's launches wait on its
+// earlier ones, so its calls can share a buffer if the launches of one call
+// follow each other: g_rosa_mu is held from the choice of the buffer to the
+// call's last launch.  The handle of the per-thread default stream stands for
+// another stream in each thread.  An outgrown buffer is not freed, since launches
+// in flight or a captured graph may still use it; the next one is at least twice
+// as large, so what a stream has outgrown is less than what it uses.  Calls under
+// capture have a buffer apart from the stream's eager calls, beside which the
+// graph may be replayed.
+using RosaScratchKey = std::tuple<int, hipStream_t, std::thread::id, bool>;
 std::mutex g_rosa_mu;
-std::map<std::pair<int, hipStream_t>, std::pair<float *, size_t>> g_rosa_scratch;
+std::map<RosaScratchKey, std::pair<float *, size_t>> g_rosa_scratch;
 
 bool op_rosa_sequential() {
     const char *e = std::getenv("YUF_ROSA_SEGMENTED");
     return e && std::strcmp(e, "0") == 0;
 }
 
-hipError_t op_rosa_scratch(hipStream_t stream, size_t floats, float **out) {
+// With g_rosa_mu held.
+hipError_t op_rosa_scratch(hipStream_t stream, bool capturing, size_t floats, float **out) {
     int dev = 0;
     hipError_t err = hipGetDevice(&dev);
     if (err != hipSuccess) return err;
-    std::lock_guard<std::mutex> lock(g_rosa_mu);
-    auto &slot = g_rosa_scratch[{dev, stream}];
+    const std::thread::id owner = stream == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
+    auto &slot = g_rosa_scratch[{dev, stream, owner, capturing}];
     if (slot.second < floats) {
-        if (slot.first) {
-            // Earlier launches on this stream may still read the old buffer.
-            if ((err = hipStreamSynchronize(stream)) != hipSuccess) return err;
-            (void)hipFree(slot.first);
-            slot = {nullptr, 0};
-        }
+        const size_t size = std::max(floats, 2 * slot.second);
+        // Allocating is no stream operation: it may happen while this or another stream is captured.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if ((err = hipThreadExchangeStreamCaptureMode(&mode)) != hipSuccess) return err;
         float *p = nullptr;
-        if ((err = hipMalloc(&p, floats * sizeof(float))) != hipSuccess) return err;
-        slot = {p, floats};
+        err = hipMalloc(&p, size * sizeof(float));
+        const hipError_t back = hipThreadExchangeStreamCaptureMode(&mode);
+        if (err != hipSuccess) return err;
+        slot = {p, size};
+        if (back != hipSuccess) return back;
     }
     *out = slot.first;
     return hipSuccess;
@@ -1168,23 +1182,23 @@ int rosa_operator(int B, int T, int D, const float *cand, const float *write, co
     } else {
         // Segments (as the engine's prefill), or one segment, which needs no
         // scratch: for ragged lengths of the no-allocation entry point (its array
-        // is shared by every stream), under capture (the graph would keep a
-        // buffer that a larger call frees) and where memory is short.
+        // is shared by every stream), for ragged lengths under capture (graphs of
+        // them may be replayed beside each other; graphs of multiples of 64 share
+        // their capture stream's buffer) and where the buffer cannot be had.
         float *buf = nullptr;
+        std::unique_lock<std::mutex> lock(g_rosa_mu, std::defer_lock);
         if (rosa_segments(T) > 1 && noalloc && bounded) {
             int rc = noalloc_scratch(&buf);
             if (rc != YUF_OK) return rc;
         } else if (rosa_segments(T) > 1 && !noalloc) {
-            const size_t need = rosa_seg_scratch(B, T, D) + (size_t)D * D;
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-            if (bounded) {
-                if ((err = op_rosa_scratch(st, need, &buf)) != hipSuccess)
-                    return fail(YUF_ERR_OOM, std::string("rosa scratch: ") + hipGetErrorString(err));
-            } else if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-                       op_rosa_scratch(st, need, &buf) != hipSuccess) {
-                (void)hipGetLastError();
+            const bool known = hipStreamIsCapturing(st, &cap) == hipSuccess;
+            const bool capturing = cap != hipStreamCaptureStatusNone;
+            lock.lock();
+            if (!known || (capturing && !bounded) ||
+                op_rosa_scratch(st, capturing, rosa_seg_scratch(B, T, D) + (size_t)D * D, &buf) != hipSuccess)
                 buf = nullptr;
-            }
+            if (!buf) (void)hipGetLastError();
         }
         err = launch_rosa_segmented(p, nullptr, buf, st);
     }
