@@ -99,11 +99,13 @@ int yuf_rosa_scan_f32(int B, int T, int D,
  * allocating call.  No counterpart in the reference; for callers that cannot
  * allocate device memory (code under HIP graph capture, serving loops and
  * harnesses that forbid hipMalloc).  Same arguments, semantics and results.
- * The segmented form (T % 64 == 0, T >= 128, D in {64, 128, 256}) keeps its
- * scratch -- D * D + 2 * B * (T / 64) * D floats -- in a static 16 MiB device
- * array (4,194,304 floats) that every GPU the library runs on holds until the
- * process ends; larger calls fail with YUF_ERR_INVALID.  Other shapes use no
- * scratch.  All calls on one GPU share that array: calls that overlap on one
+ * Calls in segments (D in {64, 128, 256}, T > 192) keep their scratch in a
+ * static 16 MiB device array (4,194,304 floats) that every GPU the library runs
+ * on holds until the process ends.  With T % 64 == 0 and T >= 128, calls with
+ * D * D + 2 * B * (T / 64) * D floats above that fail with YUF_ERR_INVALID;
+ * other lengths that do not fit run as one segment per sequence (slower, and
+ * equal to yuf_rosa_scan_f32 up to rounding).  Other shapes use no scratch.  All
+ * calls on one GPU share that array: calls that overlap on one
  * GPU (other streams, other host threads) race and must be ordered by the
  * caller.  The first call on a device resolves the array's address there
  * (hipGetSymbolAddress, not a stream operation).  YUF_ROSA_SEGMENTED does

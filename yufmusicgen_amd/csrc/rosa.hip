@@ -1148,11 +1148,12 @@ int noalloc_scratch(float **out) {
     return YUF_OK;
 }
 
-// The operator: argument checks, then the segmented form (scratch from the
-// growing per-stream buffer, or from `scratch` when noalloc) or the
-// sequential chunked scan (no scratch).  The no-allocation variant does not
-// read YUF_ROSA_SEGMENTED: its scratch capacity is checked on every call that
-// can take the segmented form, before any launch, whatever the switch says.
+// The operator: argument checks, then the segment form (scratch from the growing
+// per-stream buffer, or from `scratch` when noalloc; none for one segment) or,
+// for other D, the sequential chunked scan (no scratch).  The no-allocation
+// variant does not read YUF_ROSA_SEGMENTED: its scratch capacity is checked on
+// every multiple of 64 that can take segments, before any launch, whatever the
+// switch says.
 int rosa_operator(int B, int T, int D, const float *cand, const float *write, const float *read_raw,
                   const float *decay, const float *direction, const float *memory_in, float *memory_out,
                   float *read_out, void *stream, bool noalloc) {
@@ -1167,7 +1168,8 @@ int rosa_operator(int B, int T, int D, const float *cand, const float *write, co
     p.memory_in = memory_in; p.memory_out = memory_out; p.read_out = read_out;
     const hipStream_t st = static_cast<hipStream_t>(stream);
     hipError_t err = hipSuccess;
-    // Shapes that admit the no-allocation entry point's scratch rule.
+    // Shapes that the no-allocation entry point refuses above its documented
+    // capacity (64-token segments: never less than what the call uses).
     const bool bounded = B > 0 && T >= 128 && T % 64 == 0 && (D == 64 || D == 128 || D == 256);
     if (noalloc && bounded) {
         const size_t seg = (size_t)B * (T / 64) * D, need = (size_t)D * D + 2 * seg;
@@ -1181,22 +1183,25 @@ int rosa_operator(int B, int T, int D, const float *cand, const float *write, co
         err = launch_rosa(p, st);
     } else {
         // Segments (as the engine's prefill), or one segment, which needs no
-        // scratch: for ragged lengths of the no-allocation entry point (its array
-        // is shared by every stream), for ragged lengths under capture (graphs of
-        // them may be replayed beside each other; graphs of multiples of 64 share
-        // their capture stream's buffer) and where the buffer cannot be had.
+        // scratch: for ragged lengths under capture (graphs of them may be
+        // replayed beside each other; graphs of multiples of 64 share their
+        // capture stream's buffer), for ragged lengths of the no-allocation entry
+        // point that its array does not hold, and where the buffer cannot be had.
         float *buf = nullptr;
         std::unique_lock<std::mutex> lock(g_rosa_mu, std::defer_lock);
-        if (rosa_segments(T) > 1 && noalloc && bounded) {
-            int rc = noalloc_scratch(&buf);
-            if (rc != YUF_OK) return rc;
-        } else if (rosa_segments(T) > 1 && !noalloc) {
+        const size_t need = rosa_seg_scratch(B, T, D) + (size_t)D * D;
+        if (rosa_segments(T) > 1 && noalloc) {
+            if (bounded || need <= kNoAllocScratchFloats) {
+                int rc = noalloc_scratch(&buf);
+                if (rc != YUF_OK) return rc;
+            }
+        } else if (rosa_segments(T) > 1) {
             hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
             const bool known = hipStreamIsCapturing(st, &cap) == hipSuccess;
             const bool capturing = cap != hipStreamCaptureStatusNone;
             lock.lock();
             if (!known || (capturing && !bounded) ||
-                op_rosa_scratch(st, capturing, rosa_seg_scratch(B, T, D) + (size_t)D * D, &buf) != hipSuccess)
+                op_rosa_scratch(st, capturing, need, &buf) != hipSuccess)
                 buf = nullptr;
             if (!buf) (void)hipGetLastError();
         }
