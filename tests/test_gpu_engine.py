@@ -386,6 +386,7 @@ def test_rosa_segmented_prefill_matches_sequential(tmp_path, monkeypatch):
     ("0.1b", 4, 4 * 256, "last", "f32"),
     ("0.1b", 5, 5 * 256, "all", "f32"),   # uneven parts (1, 1, 1, 2 sequences)
     ("wide2", 4, 4 * 256, "all", "bf16"),  # the bf16-weight large-tile kernels
+    ("wide2", 5, 5 * 256, "all", "bf16"),  # 80 heads of 64: other scan forms as one part and as two or four
 ])
 def test_prefill_stream_groups_are_bit_identical(tmp_path, monkeypatch, preset, n, max_tokens, logits, weights):
     """A prefill whose parts (>= 256 rows each) run on two or four HIP streams

@@ -86,6 +86,27 @@ def test_wkv7_split_heads(size, steps, split, monkeypatch):
     np.testing.assert_allclose(s.cpu().numpy(), se.numpy(), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("size", [32, 40, 48, 64])
+@pytest.mark.parametrize("steps", [33, 80])
+def test_wkv7_forms_are_bit_identical(size, steps, monkeypatch):
+    """Whole heads, two workgroups per head and one per 16 value rows sum in one
+    order: how many heads a call brings, which chooses the form, does not change
+    the bits of a head's outputs and state."""
+    from yufmusicgen_amd.ops import rwkv7_scan
+
+    print(f"wkv7 forms N={size} T={steps}", flush=True)
+    monkeypatch.setenv("YUF_WKV7_KERNEL", "chunked")
+    arrs = wkv_inputs(900 + size + steps, 2, steps, 3, size)
+    s0 = np.random.default_rng(size).standard_normal((2, 3, size, size)).astype(np.float32) * 0.3
+    got = []
+    for split in ("0", "2", "4"):
+        monkeypatch.setenv("YUF_WKV7_SPLIT", split)
+        got.append(rwkv7_scan(*(_dev(x) for x in arrs), state=_dev(s0)))
+    torch.cuda.synchronize()
+    for y, s in got[1:]:
+        assert torch.equal(y, got[0][0]) and torch.equal(s, got[0][1])
+
+
 def test_wkv7_reference_golden(golden_dir):
     from yufmusicgen_amd.ops import rwkv7_scan
 
