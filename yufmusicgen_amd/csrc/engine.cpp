@@ -102,7 +102,8 @@ struct Engine {
     float *dl_buf = nullptr;         // per-XCD group activations
     int *dl_sync = nullptr;          // per-layer counter blocks, zeroed at the start of each step
     size_t dl_sync_ints = 0;         // per layer
-    int pass_rows = 0;  // rows of the running prefill chunk over all its parts (0: one part); sizes GEMM tiles
+    // Rows and streams of the running prefill chunk over all its parts (0: one part): size GEMM tiles and scan splits.
+    int pass_rows = 0, pass_streams = 0;
     int prefill_groups = 0;                                    // YUF_PREFILL_GROUPS=1..4: streams for the batch's parts (0: automatic)
     // The first layer's WKV-7 step launch of the last decode pass (fused
     // low-rank form), kept for yuf_engine_time_wkv_step.
@@ -613,6 +614,7 @@ int forward_pass(Engine &e, const Act &a, int n, int Tc, float *logits, int mode
         }
         WkvParams wp;
         wp.B = n; wp.T = Tc; wp.H = s.heads;
+        wp.call_heads = e.pass_streams * s.heads;
         wp.r = a.r; wp.w = a.wr; wp.k = a.k; wp.v = a.v; wp.a = a.al;
         wp.k_k = w.k_k; wp.k_a = w.k_a;
         wp.state_in = wkv; wp.state_out = wkv; wp.slot = a.slots; wp.y = a.y;
@@ -810,19 +812,20 @@ int prefill_impl(Engine &e, int n, int T, const int32_t *tokens_dev, float *logi
         // the parts before it.
         const int layers = e.s.layers;
         e.pass_rows = G > 1 ? n * tc : 0;
+        e.pass_streams = G > 1 ? n : 0;
         for (int l = 0; l == 0 || l < layers; ++l) {
             const int l1 = G > 1 ? std::min(l + 1, layers) : layers;
             for (int g = 0; g < G; ++g) {
                 const int rc = forward_pass(e, acts[g], ns[g], tc, lgs[g], chunk_mode, T, t0, l, l1);
                 if (rc != YUF_OK) {
-                    e.pass_rows = 0;
+                    e.pass_rows = e.pass_streams = 0;
                     (void)join_forked();
                     return rc;
                 }
             }
             if (l1 == layers) break;
         }
-        e.pass_rows = 0;
+        e.pass_rows = e.pass_streams = 0;
         ENG_TRY(join_forked(), "join");
         if (head_after) {
             const Act a0 = act_at(e, e.stream, 0, tc);

@@ -17,6 +17,9 @@ struct WkvParams {
     // `k` the raw key; kk = normalize(k * k_k) per head, a = -kk, b = kk * alpha,
     // k_hat = k * (1 + (alpha - 1) * k_a)  (yufmusicgen/model.py:114-122).
     const float *k_k = nullptr, *k_a = nullptr;  // [H * N]
+    // Heads of the whole call when these B H are one of several parts that run
+    // side by side (0: B H); only the choice of the scan's form reads it.
+    int call_heads = 0;
     // State [slots, H, N, N]; stream b uses slot `slot[b]` (slot == nullptr: b).
     const float *state_in = nullptr;
     float *state_out = nullptr;

@@ -51,6 +51,7 @@
 // the matching A operand is one ds_read_b128 of 4 consecutive k per lane.
 #include "common.h"
 #include "kernels.h"
+#include "wkv7_split.h"
 
 #include <cstdlib>
 #include <cstring>
@@ -735,26 +736,16 @@ hipError_t launch_nb_vt(const WkvParams &p, int N, bool prep, hipStream_t stream
     return hipGetLastError();
 }
 
-// Workgroups of a head: one per value tile where all of them run at once (one
-// fits a CU), else two, else one.  A finer split repeats the key-space stages
-// but shortens the busiest SIMD of a chunk; past one round of the 256 CUs it
-// loses.  us for 777 tokens, whole / two / one per tile: N = 64, 48 heads
-// 130 / 104 / 85, 80 heads 129 / 107 / 163, 128 heads 132 / 111 / 171, 192
-// heads 137 / 211 / 245; N = 40, 16 heads 78 / 64.9 / 63.3, 80 heads 80.6 /
-// 68.2 / 67.1, 128 heads 83 / 71 / 126.  YUF_WKV7_SPLIT forces it: 0 whole
-// heads, 1 at least two, 2 two, 4 one per tile.
-constexpr int kCus = 256;
-
+// YUF_WKV7_SPLIT forces the form: 0 whole heads, 1 at least two workgroups per
+// head, 2 two, 4 one per value tile.
 template <int NB>
 hipError_t launch_nb(const WkvParams &p, int N, bool prep, hipStream_t stream) {
     if constexpr (NB > 1) {
         constexpr int kVt2 = (NB + 1) / 2;
-        const int heads = p.B * p.H;
-        const char *e = std::getenv("YUF_WKV7_SPLIT");
-        const int force = e ? std::atoi(e) : -1;
-        const bool two_ok = !(prep && op_only(NB, kVt2));
-        if (force == 4 || (force != 0 && force != 2 && heads * NB <= kCus)) return launch_nb_vt<NB, 1>(p, N, prep, stream);
-        if (two_ok && force != 0 && (force > 0 || heads * 2 <= kCus)) return launch_nb_vt<NB, kVt2>(p, N, prep, stream);
+        const int vt = wkv7_value_tiles(NB, p.B * p.H, p.call_heads, !(prep && op_only(NB, kVt2)),
+                                        std::getenv("YUF_WKV7_SPLIT"));
+        if (vt == 1) return launch_nb_vt<NB, 1>(p, N, prep, stream);
+        if (vt == kVt2) return launch_nb_vt<NB, kVt2>(p, N, prep, stream);
     }
     return launch_nb_vt<NB, 0>(p, N, prep, stream);
 }
