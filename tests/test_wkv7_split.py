@@ -16,6 +16,7 @@ pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not ava
 MAIN = r"""
 #include "wkv7_split.h"
 #include <cstdio>
+#include <cstdlib>
 int main(int argc, char **argv) {
     for (int i = 1; i + 4 < argc; i += 5)
         std::printf("%d\n", yuf::wkv7_value_tiles(std::atoi(argv[i]), std::atoi(argv[i + 1]), std::atoi(argv[i + 2]),
@@ -55,6 +56,7 @@ def test_form_follows_the_heads_that_run_at_once(value_tiles, nb, heads, call, t
 @pytest.mark.parametrize("nb,heads,two,force,want", [
     (3, 16, True, "0", 0), (3, 1000, True, "1", 2), (3, 16, True, "1", 1), (3, 16, True, "2", 2), (3, 1000, True, "4", 1),
     (4, 16, False, "2", 0), (4, 1000, False, "1", 0), (4, 1000, False, "4", 1),
+    (3, 1000, True, "on", 2), (3, 1000, True, "true", 2), (3, 16, True, "", 1), (3, 1000, True, "00", 2),
 ])
 def test_forced_forms(value_tiles, nb, heads, two, force, want):
     assert value_tiles(nb, heads, 0, two, force) == want

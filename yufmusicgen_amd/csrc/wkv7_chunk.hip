@@ -736,8 +736,8 @@ hipError_t launch_nb_vt(const WkvParams &p, int N, bool prep, hipStream_t stream
     return hipGetLastError();
 }
 
-// YUF_WKV7_SPLIT forces the form: 0 whole heads, 1 at least two workgroups per
-// head, 2 two, 4 one per value tile.
+// YUF_WKV7_SPLIT forces the form: 0 whole heads, 2 two workgroups per head, 4 one
+// per value tile, any other text at least two.
 template <int NB>
 hipError_t launch_nb(const WkvParams &p, int N, bool prep, hipStream_t stream) {
     if constexpr (NB > 1) {

@@ -1,8 +1,6 @@
 // How the chunked WKV-7 scan spreads heads over workgroups: host arithmetic only.
 #pragma once
 
-#include <cstdlib>
-
 namespace yuf {
 
 constexpr int kWkvCus = 256;  // workgroups of the scan that run at once: one fits a CU
@@ -22,7 +20,9 @@ constexpr int kWkvCus = 256;  // workgroups of the scan that run at once: one fi
 // (2 layers, 1111 tokens, whole / one per tile: 96 heads in four 2200 / 2040, 128
 // in four 2440 / 2375, 192 in two 2370 / 2550).
 inline int wkv7_value_tiles(int NB, int heads, int all, bool two, const char *force) {
-    const int forced = force ? std::atoi(force) : -1;
+    // Of the forcing texts "0", "2" and "4" name a form; any other one means split.
+    int forced = -1;
+    if (force) forced = (force[0] == '0' || force[0] == '2' || force[0] == '4') && !force[1] ? force[0] - '0' : 1;
     if (NB < 2 || forced == 0) return 0;
     const int pair = (NB + 1) / 2;
     if (forced == 4) return 1;
