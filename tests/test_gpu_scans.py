@@ -284,6 +284,29 @@ def test_rosa_segments(dim, steps):
         np.testing.assert_allclose(mem.cpu().numpy(), me.numpy(), rtol=RTOL, atol=ATOL)
 
 
+@pytest.mark.parametrize("dim", [64, 128, 256])
+@pytest.mark.parametrize("steps", [33, 705])
+def test_rosa_nearly_closed_write_gates(dim, steps):
+    """Write gates down to sigmoid(-80) (1e-35) with saturated candidates: the
+    inputs stay what they are instead of vanishing, so reads and memory follow
+    the float64 oracle to 3e-5 of their largest value (e^{-80} in fp32 is good to
+    |w| 2^-23 = 1e-5; the state is a sum of such values, 1e3 and more above the
+    smallest normal number)."""
+    from yufmusicgen_amd.ops import rosa_householder_scan
+
+    print(f"rosa closed gates D={dim} T={steps}", flush=True)
+    cand, write, read_raw, decay, u = rosa_inputs(91 + dim, 2, steps, dim)
+    cand = np.sign(cand + 0.01).astype(np.float32) * 12.0
+    write = (-70.0 - 10.0 * np.random.default_rng(4).random(write.shape)).astype(np.float32)
+    args = [cand, write, read_raw, decay, u, np.zeros((2, dim), dtype=np.float32)]
+    out, mem = rosa_householder_scan(*(_dev(x) for x in args), gated=False)
+    torch.cuda.synchronize()
+    re, me = orosa.rosa_scan(*(torch.from_numpy(np.asarray(x)).double() for x in args), gated=False)
+    for got, want in ((out, re), (mem, me)):
+        assert float(want.abs().max()) > 1e-32
+        assert float((got.cpu().double() - want).abs().max()) <= 3e-5 * float(want.abs().max())
+
+
 def _rosa_call(args, mem, out, gated, stream):
     from yufmusicgen_amd._lib import check, lib
 

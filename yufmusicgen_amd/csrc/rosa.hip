@@ -553,11 +553,12 @@ __device__ __forceinline__ float recip(float x) {
     return x > 0x1p126f ? r : fmaf(fmaf(-x, r, 1.0f), r, r);
 }
 __device__ __forceinline__ float seg_gate(float x) { return recip(1.0f + __expf(-x)); }
-// tanh(x) sigmoid(w) = (E - 1) / ((E + 1) (1 + F)), E = e^{2x}, F = e^{-w}: one
-// reciprocal.  tanh is 1 in fp32 from x = 10 on (the comparison keeps NaN); 0 for x = 0.
+// tanh(x) sigmoid(w) = sign(x) (1 - E) / ((1 + E) (1 + F)), E = e^{-2|x|} <= 1, F =
+// e^{-w}: one reciprocal, whose argument is finite down to w = -88 (with e^{2x} in
+// it, it overflowed and the result vanished below w = -69).
 __device__ __forceinline__ float seg_cand(float x, float w) {
-    const float E = __expf(2.0f * (x > 10.0f ? 10.0f : x));
-    return (E - 1.0f) * recip((E + 1.0f) * (1.0f + __expf(-w)));
+    const float E = __expf(-2.0f * fabsf(x));
+    return copysignf((1.0f - E) * recip((1.0f + E) * (1.0f + __expf(-w))), x);
 }
 
 // Sum over aligned groups of G lanes (8 or 16), every lane gets it.
