@@ -965,3 +965,27 @@ def test_time_wkv_step_leaves_the_state_alone(tmp_path):
         eng.close()
     for a, b in zip(outs[0], outs[1]):
         np.testing.assert_array_equal(a, b)
+
+
+def test_decode_with_low_rank_planes_far_apart(tmp_path):
+    """The rank-L rows' planes are max_tokens rows apart: at 4.3 M tokens and L =
+    128 the third one starts 4.4 GB behind the first, beyond 32-bit offsets (an
+    engine of 18 GB).  Decode steps equal those of a small engine bit for bit."""
+    import dataclasses
+
+    class Rank128(ModelConfig):
+        low_rank = 128
+
+    cfg = Rank128(**dataclasses.asdict(dataclasses.replace(PRESETS["state_test"], rosa_size=8)))
+    path = tmp_path / "m.yuf"
+    write_yuf(path, cfg, synth_weights(cfg, seed=8))
+    ck = Checkpoint.load(path)
+    tokens = uniform_tokens(4, 3, 6, cfg.vocab_size)
+    outs = []
+    for max_tokens in (64, 4_300_000):
+        print(f"far low-rank planes max_tokens={max_tokens}", flush=True)
+        eng = Engine(ck, max_streams=3, max_tokens=max_tokens)
+        outs.append((np.stack([eng.step(tokens[:, t]) for t in range(6)]), _states_from_blob(eng, [0, 1, 2])))
+        eng.close()
+    for a, b in zip(*outs):
+        np.testing.assert_array_equal(a, b)

@@ -384,8 +384,7 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
         // staged in 62 KB of LDS).  N % 8 == 0: m is uniform over a wave.
         constexpr int kT = kStepThreads * SPW;
         constexpr int kDl = 8, kI = kStepLrMaxL / (4 * kDl), kP = (3 * N * kDl + kT - 1) / kT;
-        constexpr int kL1 = (SPW * 3 * kStepLrMaxL + kT - 1) / kT;
-        static_assert(N % 8 == 0 && SPW <= kDl, "dot layout");
+        static_assert(N % 8 == 0 && SPW <= kDl && SPW * kStepLrMaxL <= kT, "dot layout; a thread per rank-L value of a plane");
         const int L = p.L, flat = threadIdx.x, dl = flat % kDl;
         float4 wreg[kP][kI];
 #pragma unroll
@@ -399,25 +398,20 @@ __global__ void __launch_bounds__(kStepThreads * SPW) wkv7_step_kernel(WkvParams
                 wreg[ps][i] = buf_load4(rw, j < L ? (uint32_t)(c * L + j) * 4u : kBufferOob);
             }
         }
-        const auto rlr = make_rsrc(p.lr, (uint32_t)((2 * p.lr_plane + (size_t)p.B * L) * 4));
-        float lreg[kL1];
+        // A descriptor per plane of the rank-L rows: planes are max_tokens * L floats
+        // apart, which one descriptor's 32-bit offsets need not span.
+        const int sb = flat / L, lj = flat - sb * L, lrow = (blockIdx.x / p.H) * SPW + sb;
+        const uint32_t loff = sb < SPW && lrow < p.B ? (uint32_t)(lrow * L + lj) * 4u : kBufferOob;
+        float lreg[3];
 #pragma unroll
-        for (int i = 0; i < kL1; ++i) {
-            const int e = flat + i * kT;
-            const int sb = e / (3 * L), rem = e - sb * 3 * L, m = rem / L, j = rem - m * L;
-            const int b2 = (blockIdx.x / p.H) * SPW + sb;
-            const bool ok = sb < SPW && b2 < p.B;
-            lreg[i] = buf_load(rlr, (((uint32_t)m * (uint32_t)p.lr_plane + (uint32_t)(b2 * L + j)) * 4u) | (ok ? 0u : kBufferOob));
-        }
+        for (int m = 0; m < 3; ++m)
+            lreg[m] = buf_load(make_rsrc(p.lr + m * p.lr_plane, (uint32_t)(p.B * L) * 4u), loff);
         const float w0c = buf_load(make_rsrc(p.w0 + h * N, N * 4), col ? (uint32_t)tid * 4u : kBufferOob);
         const float a0c = buf_load(make_rsrc(p.a0 + h * N, N * 4), col ? (uint32_t)tid * 4u : kBufferOob);
         load_state();
 #pragma unroll
-        for (int i = 0; i < kL1; ++i) {
-            const int e = flat + i * kT;
-            const int sb = e / (3 * L), rem = e - sb * 3 * L, m = rem / L, j = rem - m * L;
-            if (sb < SPW) lrs[sb][m][j] = lreg[i];
-        }
+        for (int m = 0; m < 3; ++m)
+            if (sb < SPW) lrs[sb][m][lj] = lreg[m];
         ksq = wave_sum((kv * kk) * (kv * kk));
         lds_barrier();
 #pragma unroll
