@@ -190,19 +190,19 @@ def test_c1_tiny_greedy_256_steps_vs_oracle(tmp_path):
     np.testing.assert_allclose(_states_from_blob(eng, [0]), state_to_blob(state), rtol=1e-4, atol=1e-4)
 
 
-@pytest.mark.parametrize("steps", [80, 160, 256])
-def test_default_model_short_prefill_and_decode_vs_oracle(tmp_path, steps):
+@pytest.mark.parametrize("steps,max_tokens", [(80, 256), (160, 256), (256, 256), (700, 700)])
+def test_default_model_short_prefill_and_decode_vs_oracle(tmp_path, steps, max_tokens):
     """The 0.1B architecture (14L, d=640, 16x40, ROSA 128, V=20480) on a short
     batch, prefill then decode, against the float64 oracle.  2 x 160 tokens
-    put every prefill product on the 256-row GEMM tiles; 2 x 256 tokens run as
-    two 128-token chunks whose ROSA scans take the segmented path (64-token
-    segments), the second from the carried state."""
+    have more than 256 rows in every prefill product; 2 x 256 tokens run as two
+    128-token chunks, the second from the carried state, and 2 x 700 as two
+    350-token ones whose ROSA scans run in 64-token segments, the last one ragged."""
     cfg = PRESETS["0.1b"]
     weights = synth_weights(cfg, seed=0)
     path = tmp_path / "m.yuf"
     write_yuf(path, cfg, weights)
     tokens = prompt_tokens(1, 2, steps, cfg.vocab_size)
-    eng = Engine(Checkpoint.load(path), max_streams=2, max_tokens=256)
+    eng = Engine(Checkpoint.load(path), max_streams=2, max_tokens=max_tokens)
     got = eng.prefill(tokens, logits="all")
     oracle = OracleModel(cfg.to_dict(), weights)
     ref, state = oracle.forward(tokens)
@@ -359,25 +359,65 @@ def test_bf16_checkpoint_equals_rounded_f32_checkpoint(tmp_path):
     assert np.abs(outs["f32file-f32"][0] - outs["bf16file-f32"][0]).max() > 0
 
 
-def test_rosa_segmented_prefill_matches_sequential(tmp_path, monkeypatch):
-    """The segmented ROSA prefill (parallel 64-token segments around an A^64
-    carry pass) against the sequential chunked scan, through the whole model:
-    logits and states, with a carried state and a decode step after it."""
+@pytest.mark.parametrize("head,tail", [(192, 128), (320, 333), (705, 1030)])
+def test_rosa_segmented_prefill_matches_sequential(tmp_path, monkeypatch, head, tail):
+    """The segment form of the ROSA prefill against the sequential chunked scan,
+    through the whole model with slow decays (lambda = 0.99, so that a segment's
+    start state matters in the next ones): logits and states, with a carried state
+    and a decode step after it.  192 and 128 tokens run as one segment, 320 and 333
+    in 64-token segments around A^64 (the last one whole and ragged), 705 and 1030
+    in ragged 64- and 128-token ones (A^128)."""
     cfg = PRESETS["0.1b"]
     path = tmp_path / "m.yuf"
-    write_yuf(path, cfg, synth_weights(cfg, seed=5))
+    weights = synth_weights(cfg, seed=5)
+    for name in weights:
+        if name.endswith("rosa.decay"):
+            weights[name] = np.full_like(weights[name], 4.6)
+    write_yuf(path, cfg, weights)
     ck = Checkpoint.load(path)
-    tokens = uniform_tokens(9, 3, 320, cfg.vocab_size)
+    tokens = uniform_tokens(9, 3, head + tail, cfg.vocab_size)
     outs = []
     for seg in ("1", "0"):
+        print(f"rosa segmented prefill {head} + {tail} segmented={seg}", flush=True)
         monkeypatch.setenv("YUF_ROSA_SEGMENTED", seg)
-        eng = Engine(ck, max_streams=3, max_tokens=3 * 192)
-        head = eng.prefill(tokens[:, :192], logits="all")
-        tail = eng.prefill(tokens[:, 192:], logits="all")  # 128 tokens from the carried state
+        eng = Engine(ck, max_streams=3, max_tokens=3 * max(head, tail))
+        first = eng.prefill(tokens[:, :head], logits="all")
+        rest = eng.prefill(tokens[:, head:], logits="all")  # from the carried state
         nxt = eng.step(tokens[:, 0])
-        outs.append((head, tail, nxt, _states_from_blob(eng, [0, 1, 2])))
+        outs.append((first, rest, nxt, _states_from_blob(eng, [0, 1, 2])))
+        eng.close()
     for a, b in zip(outs[0], outs[1]):
         np.testing.assert_allclose(a, b, rtol=1e-4, atol=1e-4)
+
+
+def test_rosa_carry_pass_in_prefill_parts(tmp_path, monkeypatch):
+    """4200 tokens in one pass: 33 segments, above the number whose carry the
+    second launch walks, so that the separate carry pass runs, in two parts with
+    scratch of their own.  Against one part bit for bit, the sequential scan and
+    the float64 oracle (the part with the larger scratch offset), lambda = 0.99."""
+    cfg = ModelConfig(vocab_size=300, d_model=64, n_layers=2, n_heads=4, head_size=16, rosa_size=64)
+    weights = synth_weights(cfg, seed=15)
+    for name in weights:
+        if name.endswith("rosa.decay"):
+            weights[name] = np.full_like(weights[name], 4.6)
+    path = tmp_path / "m.yuf"
+    write_yuf(path, cfg, weights)
+    ck = Checkpoint.load(path)
+    tokens = uniform_tokens(16, 2, 4200, cfg.vocab_size)
+    outs = {}
+    for groups, seg in (("2", "1"), ("1", "1"), ("2", "0")):
+        print(f"rosa carry pass groups={groups} segmented={seg}", flush=True)
+        monkeypatch.setenv("YUF_PREFILL_GROUPS", groups)
+        monkeypatch.setenv("YUF_ROSA_SEGMENTED", seg)
+        eng = Engine(ck, max_streams=2, max_tokens=2 * 4200)
+        outs[groups + seg] = (eng.prefill(tokens, logits="all"), _states_from_blob(eng, [0, 1]))
+        eng.close()
+    for a, b, c in zip(outs["21"], outs["11"], outs["20"]):
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_allclose(a, c, rtol=1e-4, atol=1e-4)
+    ref, state = OracleModel(cfg.to_dict(), weights).forward(tokens[1:])
+    np.testing.assert_allclose(outs["21"][0][1], ref.numpy()[0], rtol=0, atol=LOGIT_ATOL)
+    np.testing.assert_allclose(outs["21"][1][1], state_to_blob(state)[0], rtol=1e-4, atol=1e-4)
 
 
 @pytest.mark.parametrize("preset,n,max_tokens,logits,weights", [

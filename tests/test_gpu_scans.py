@@ -220,11 +220,12 @@ def test_rosa_full_size(decay_value):
     np.testing.assert_allclose(m.cpu().numpy(), me.numpy(), rtol=RTOL, atol=ATOL)
 
 
-@pytest.mark.parametrize("dim,steps,gated", [(64, 128, True), (128, 640, False), (256, 256, True), (128, 2048, True)])
+@pytest.mark.parametrize("dim,steps,gated", [(64, 128, True), (64, 320, True), (128, 640, False), (256, 256, True),
+                                             (256, 1088, False), (128, 2048, True)])
 def test_rosa_segmented_operator(dim, steps, gated, monkeypatch):
-    """The operator's segmented form (T a multiple of 64, T >= 128, D in {64,
-    128, 256}: A^64 built on the device in double, segments from zero, the
-    carry chain, segments from their starts) against the float64 oracle and
+    """The operator's segment form (D in {64, 128, 256}: one segment up to 192
+    tokens; above, A^64 or A^128 built on the device in double, segments from
+    zero, then each from its start state) against the float64 oracle and
     against the sequential scan (YUF_ROSA_SEGMENTED=0), from a non-zero memory."""
     from yufmusicgen_amd.ops import rosa_householder_scan
 
