@@ -24,7 +24,7 @@ ALLOWED_SCRATCH = {
     # The unsplit N = 64 chunk scan with fused prep (the C5 shape): its
     # 10-wave workgroup (three waves on some SIMDs) leaves 168 VGPRs per lane,
     # and the compiler spills 4.
-    r"wkv7_chunk_kernelILi4ELb1ELb0ELb[01]E": 20,
+    r"wkv7_chunk_kernelILi4ELb1ELb[01]ELi0E": 20,
 }
 
 
@@ -39,8 +39,8 @@ def resources():
 
 def test_report_covers_every_kernel_family(resources):
     assert len(resources) > 100
-    for family in ("gemm_big_kernel", "gemm_decode_kernel", "wkv7_chunk_kernel", "wkv7_step_kernel",
-                   "rosa_scan_kernel", "rosa_carry_kernel", "sample_kernel", "layernorm_kernel"):
+    for family in ("gemm_big_kernel", "gemm_ps_kernel", "gemm_decode_kernel", "wkv7_chunk_kernel", "wkv7_step_kernel",
+                   "rosa_scan_kernel", "rosa_seg_kernel", "rosa_carry_kernel", "sample_kernel", "layernorm_kernel"):
         assert any(family in k for k in resources), family
     for name, r in resources.items():
         for field in ("vgprs", "scratch_bytes_per_lane", "waves_per_simd", "lds_bytes", "dynamic_stack"):

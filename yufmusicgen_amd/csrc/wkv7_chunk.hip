@@ -171,11 +171,11 @@ template <int NB, int VT> struct RoleMap {
 // over the keys takes k-steps r = 0, 1 only on that tile (k-step r of lane
 // group g: key 2 g + r of the tile) instead of four k-steps of which half
 // would multiply zeros.
-template <int NB, bool PREP, bool SPLIT, bool HALF, int VT>
+template <int NB, bool PREP, bool HALF, int VT>
 __global__ void __launch_bounds__((RoleMap<NB, VT>::kWaves) * kWave)
     wkv7_chunk_kernel(WkvParams p, int N, int units, int per_xcd) {
     using Ly = Lds<NB, VT>;
-    static_assert(SPLIT == (VT > 0), "VT value tiles of a split head");
+    constexpr bool SPLIT = VT > 0;
     constexpr int NP = Ly::NP, SA = Ly::SA, kRA = Ly::kRA, kRV = Ly::kRV, kRG = Ly::kRG;
     constexpr int kExtra = SPLIT ? 1 : 0;  // iterations after the consumers' last chunk (the Y wave's)
     __shared__ __attribute__((aligned(16))) float lds[Ly::kFloats];
@@ -713,11 +713,11 @@ void launch_nb_form(const WkvParams &p, int N, bool prep, int units, int per_xcd
     const dim3 grid(per_xcd * kXcds), block(RoleMap<NB, VT>::kWaves * kWave);
     if constexpr (!op_only(NB, VT)) {
         if (prep) {
-            hipLaunchKernelGGL((wkv7_chunk_kernel<NB, true, (VT > 0), HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
+            hipLaunchKernelGGL((wkv7_chunk_kernel<NB, true, HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
             return;
         }
     }
-    hipLaunchKernelGGL((wkv7_chunk_kernel<NB, false, (VT > 0), HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
+    hipLaunchKernelGGL((wkv7_chunk_kernel<NB, false, HALF, VT>), grid, block, 0, stream, p, N, units, per_xcd);
 }
 
 // Half-padded last key tile (N % 16 == 8) unless YUF_WKV7_HALF=0.
