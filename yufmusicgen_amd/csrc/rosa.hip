@@ -501,7 +501,8 @@ __global__ void __launch_bounds__(D * D / 64) rosa_carry_kernel(int P, const flo
 // are 32 dot products over the channels (summed in double by all waves at
 // once), p = L f one small triangular product, and the states and reads follow
 // per channel.  f_1 of a chunk is p_33 of the one before.  Five barriers and
-// ~1 us per 32 tokens, against ~3 us per 16 in rosa_scan_kernel.
+// 2.2, 2.8 and 4.2 us per 32 tokens of one segment at D = 64, 128 and 256, against
+// 3.5, 6.3 and 9.1 in rosa_scan_kernel.
 //
 // Long sequences are cut into segments of L tokens: one launch runs every
 // segment but the last to its end state (the first from the true start, the
