@@ -548,18 +548,21 @@ struct SegCfg {
     static constexpr int kLds = kSegC * PS * 8 + 2 * kSegC * D * 4;  // partial products, e, gates
 };
 
-// 1 / x to within a rounding or two, x >= 1 or NaN: inf gives 0.
+// 1 / x to within a rounding or two, x >= 2^-30 or NaN: inf gives 0.
 __device__ __forceinline__ float recip(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
     return x > 0x1p126f ? r : fmaf(fmaf(-x, r, 1.0f), r, r);
 }
 __device__ __forceinline__ float seg_gate(float x) { return recip(1.0f + __expf(-x)); }
-// tanh(x) sigmoid(w) = sign(x) (1 - E) / ((1 + E) (1 + F)), E = e^{-2|x|} <= 1, F =
-// e^{-w}: one reciprocal, whose argument is finite down to w = -88 (with e^{2x} in
-// it, it overflowed and the result vanished below w = -69).
+// tanh(x) sigmoid(w) = (E - 1) / ((E + 1) (1 + F)), E = e^{2x}, F = e^{-w}: one
+// reciprocal.  tanh is 1 in fp32 from x = 10 on (the comparison keeps NaN); 0 for x = 0.
+// Both E + 1 and E - 1 carry a factor 2^-30, which changes no bit of the quotient
+// and keeps the product finite for every finite F (without it the result vanished
+// below w = -69).
 __device__ __forceinline__ float seg_cand(float x, float w) {
-    const float E = __expf(-2.0f * fabsf(x));
-    return copysignf((1.0f - E) * recip((1.0f + E) * (1.0f + __expf(-w))), x);
+    constexpr float s = 0x1p-30f;
+    const float E = __expf(2.0f * (x > 10.0f ? 10.0f : x));
+    return fmaf(E, s, -s) * recip(fmaf(E, s, s) * (1.0f + __expf(-w)));
 }
 
 // Sum over aligned groups of G lanes (8 or 16), every lane gets it.
