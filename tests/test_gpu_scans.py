@@ -260,10 +260,10 @@ def test_rosa_chunked_continuation():
 
 
 @pytest.mark.parametrize("dim", [64, 128, 256])
-@pytest.mark.parametrize("steps", [2, 31, 33, 192, 193, 320, 641, 1111, 4161])
+@pytest.mark.parametrize("steps", [2, 8, 9, 31, 33, 192, 193, 320, 641, 1111, 4161])
 def test_rosa_segments(dim, steps):
-    """The segment kernel at the edges of its 32-token chunks and of its segment
-    rule (one segment up to 192 tokens, 64- then 128-token segments with a ragged
+    """The segment kernel at the edges of its range (above 8 tokens at D = 256), of
+    its 32-token chunks and of its segment rule (one segment up to 192 tokens, 64- then 128-token segments with a ragged
     last one, the separate carry pass above 32 segments), gated and not, against
     the float64 oracle, with the memory updated in place."""
     from yufmusicgen_amd._lib import check, lib

@@ -1184,7 +1184,11 @@ int rosa_operator(int B, int T, int D, const float *cand, const float *write, co
                                              "the static buffer holds " + std::to_string(kNoAllocScratchFloats) +
                                              " -- split the batch or use yuf_rosa_scan_f32");
     }
-    if (B <= 0 || T <= 0 || !rosa_seg_ok(T, D) || (!noalloc && op_rosa_sequential())) {
+    // Up to 8 tokens of D = 256 are two of the sequential scan's chunks (8.2 us,
+    // 9.9 as one 32-token chunk; 9 tokens 10.7 / 10.1; the engine, which would launch
+    // the gates apart for it, keeps the segment kernel).
+    const bool few = D == 256 && T <= 8;
+    if (B <= 0 || T <= 0 || !rosa_seg_ok(T, D) || few || (!noalloc && op_rosa_sequential())) {
         err = launch_rosa(p, st);
     } else {
         // Segments (as the engine's prefill), or one segment, which needs no
