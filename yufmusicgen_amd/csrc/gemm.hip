@@ -38,6 +38,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "gemm_tiles.h"
 #include "kernels.h"
 
 namespace yuf {
@@ -851,7 +852,6 @@ __global__ void __launch_bounds__(kBigThreads) gemm_x3p_kernel(GemmGroup g, int 
 // products below 256 rows (100 x 640 x 640: 62 -> 8 us; X3 took 10, its split
 // being the larger part of a lone wave's step).
 // ---------------------------------------------------------------------------
-enum PsMode : int { PS_X3P = 0, PS_X3 = 1, PS_BF16 = 2, PS_F32 = 3 };
 
 template <int MODE, int BM, int BN, int WM, int WNS, int ST, int PIPE, bool STAGED>
 __global__ void __launch_bounds__(64 * WM * WNS) gemm_ps_kernel(GemmGroup g, int per_xcd) {
@@ -2038,26 +2038,6 @@ bool use_x3(const GemmGroup &g, int n) {
     return true;
 }
 
-// A tile shape and the measured time (us) of one 32-k step of it: of tiles that
-// have their CUs to themselves, and of each full round of 256 tiles.
-struct TileCost {
-    int id, bm, bn;
-    float alone, round;
-};
-// gemm_ps_kernel's tiles per mode.
-constexpr TileCost kPsTiles[4][4] = {
-    {{1, 32, 32, 0.30f, 0.168f}, {2, 64, 64, 0.60f, 0.45f}, {3, 128, 128, 1.22f, 1.25f}, {}},                        // PS_X3P
-    {{1, 32, 32, 0.35f, 0.20f}, {2, 64, 64, 0.70f, 0.48f}, {3, 128, 128, 1.65f, 1.65f}, {}},                         // PS_X3
-    {{1, 32, 32, 0.23f, 0.10f}, {2, 64, 64, 0.32f, 0.205f}, {3, 128, 128, 0.64f, 0.65f}, {4, 64, 128, 0.47f, 0.34f}},  // PS_BF16
-    {{1, 32, 32, 0.24f, 0.195f}, {2, 64, 64, 0.67f, 0.55f}, {5, 32, 64, 0.40f, 0.33f}, {}},                          // PS_F32
-};
-// The 256-row tiles of the same forms (64-wide X3P: 64-row tiles), widths 256, 160, 128, 64.
-constexpr TileCost kBigTiles[3][4] = {
-    {{0, 256, 256, 3.55f, 4.65f}, {0, 256, 160, 2.4f, 3.0f}, {0, 256, 128, 2.05f, 2.6f}, {0, 64, 64, 0.53f, 0.9f}},
-    {{0, 256, 256, 4.1f, 5.4f}, {0, 256, 160, 2.8f, 3.5f}, {0, 256, 128, 2.3f, 2.9f}, {0, 256, 64, 1.9f, 2.2f}},
-    {{0, 256, 256, 1.6f, 1.95f}, {0, 256, 160, 1.2f, 1.7f}, {0, 256, 128, 1.05f, 1.6f}, {0, 256, 64, 0.87f, 1.5f}},
-};
-
 template <int MODE, bool STAGED>
 void launch_ps_tile(const GemmGroup &g, int id, int per_xcd, dim3 grid, hipStream_t stream) {
     const dim3 b4(256), b8(512);
@@ -2106,18 +2086,13 @@ hipError_t launch_ps(GemmGroup &g, int n, int mode, const TileCost &t, hipStream
     return hipGetLastError();
 }
 
-// The tile of gemm_ps_kernel a group takes, or nullptr: it takes the 256-row
-// tiles of width big_bn (0: it has none and falls back to another kernel).
-// The estimate of a launch is its rounds of 256 tiles times the measured time
-// of a k step; tiles are counted over the rows of the whole call, since a
-// prefill's parts run side by side.  (X3P, us, this kernel against the 256-row
-// tiles: 333 x 640 x 640 9 / 50, 333 x 640 x 2560 26 / 183, 1000 x 5120 x 640 45 / 76,
-// 4096 x 5120 x 640 131 / 164; 16384 x 5120 x 640 503 / 468 keeps the latter.)
-// X3P products with K <= 128 move to it below 2048 rows only: there the output
-// write bounds both (640 x 128: 6.3 / 8.1 at 1000 rows, 11 / 9.8 at 4096).
+// The tile of gemm_ps_kernel a group takes (ps_tile_rule), or nullptr: its
+// layouts do not fit, or it takes the large tiles of width big_bn (0: it has
+// none and falls back to another kernel).
 const TileCost *ps_tile(const GemmGroup &g, int n, int mode, int big_bn) {
-    bool silu = false, n128 = true;
-    int K = 0, rows = 0;
+    bool silu = false;
+    int K = 0;
+    TileProduct shapes[kMaxGroup];
     for (int i = 0; i < n; ++i) {
         const GemmParams &p = g.p[i];
         const void *w = mode == PS_BF16 ? (const void *)p.Wh : (const void *)p.W;
@@ -2126,32 +2101,10 @@ const TileCost *ps_tile(const GemmGroup &g, int n, int mode, int big_bn) {
                            : (p.ldw % (mode == PS_BF16 ? 8 : 4) != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0))
             return nullptr;
         silu = silu || p.silu_pair;
-        n128 = n128 && p.N % 128 == 0;
         K = std::max(K, p.K);
-        rows = std::max(rows, std::max(p.rows, p.M));
+        shapes[i] = {std::max(p.rows, p.M), p.N};
     }
-    if (mode == PS_X3P && K <= 128 && rows >= 2048 && big_bn) return nullptr;
-    const auto cost = [&](const TileCost &t) {
-        long long tiles = 0;
-        for (int i = 0; i < n; ++i)
-            tiles += (long long)((std::max(g.p[i].rows, g.p[i].M) + t.bm - 1) / t.bm) * ((g.p[i].N + t.bn - 1) / t.bn);
-        if (tiles <= 256) return t.alone >= t.round ? t.alone : t.alone + (t.round - t.alone) * (float)tiles / 256.0f;
-        return std::max(t.alone, t.round * (float)((tiles + 255) / 256));
-    };
-    const TileCost *best = nullptr;
-    float least = 0.0f;
-    if (big_bn && mode != PS_F32)
-        for (const TileCost &t : kBigTiles[mode])
-            if (t.bn == big_bn) least = cost(t);
-    for (const TileCost &t : kPsTiles[mode]) {
-        if (!t.id || (silu && t.bn < 64) || (t.bn == 128 && !n128)) continue;
-        const float c = cost(t);
-        if (least == 0.0f || c < least) {
-            least = c;
-            best = &t;
-        }
-    }
-    return best;
+    return ps_tile_rule(shapes, n, K, mode, big_bn, silu);
 }
 
 template <int NT, int MI, int PRO, bool WB, int S>
