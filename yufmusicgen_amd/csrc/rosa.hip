@@ -560,7 +560,8 @@ __device__ __forceinline__ float seg_gate(float x) { return recip(1.0f + __expf(
 // and keeps the product finite for every finite F (without it the result vanished
 // below w = -69).
 __device__ __forceinline__ float seg_cand(float x, float w) {
-    constexpr float s = 0x1p-30f;
+    float s;  // 2^-30 in a scalar register (a vector one is a spill at D = 256)
+    asm("s_mov_b32 %0, 0x30800000" : "=s"(s));
     const float E = __expf(2.0f * (x > 10.0f ? 10.0f : x));
     return fmaf(E, s, -s) * recip(fmaf(E, s, s) * (1.0f + __expf(-w)));
 }

@@ -704,8 +704,7 @@ __global__ void __launch_bounds__((RoleMap<NB, VT>::kWaves) * kWave)
 }
 
 // The nine waves of the N = 64 pair form leave 168 VGPRs, which the fused prep
-// does not fit (it spills); prefills of as many heads run whole heads beside
-// their other parts' kernels anyway.
+// does not fit (it spills): the model's prefills choose between the other two.
 constexpr bool op_only(int NB, int VT) { return NB == 4 && VT == 2; }
 
 template <int NB, int VT, bool HALF>
